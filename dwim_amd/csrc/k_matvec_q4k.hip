@@ -18,9 +18,17 @@ static const float *normalized(dwim_dev *dev, const float *x, const float *norm,
     return xn && launch_rmsnorm(dev->stream, xn, x, norm, n, cols, eps) == hipSuccess ? xn : nullptr;
 }
 
+// Q4_K products may be in place.  The kernel of 5 to 64 tokens reads x while
+// other workgroups write results; the int8 kernels and the GEMM read it in a
+// launch of its own first, so products in place go to those (runs of four
+// tokens below kGemmInPlace, whose rows are read before they are written).
+constexpr size_t kGemmInPlace = 16;
+static bool by_rows(size_t n, const float *out, const float *x) { return n >= kRowsQ4kTokens && n < kGemmTokens && out != x; }
+static bool by_gemm(size_t n, const float *out, const float *x) { return n >= (out == x ? kGemmInPlace : kGemmTokens); }
+
 hipError_t launch_matvec_q4k(dwim_dev *dev, const dwim_weight *w, float *out, const float *x, size_t n, int add) {
-    if (n >= kRowsQ4kTokens && n < kGemmTokens) return launch_rows(dev, w, nullptr, out, x, n, add);
-    if (n >= kGemmTokens) return launch_gemm_q4k(dev, w, out, x, n, add);
+    if (by_rows(n, out, x)) return launch_rows(dev, w, nullptr, out, x, n, add);
+    if (by_gemm(n, out, x)) return launch_gemm_q4k(dev, w, out, x, n, add);
     return launch_mv_q4k_mfma_tokens(dev, &w, &out, &add, 1, 0, x, n, nullptr, 0.0f, nullptr);
 }
 
@@ -51,11 +59,11 @@ hipError_t launch_matvec_q4k_multi(dwim_dev *dev, const dwim_weight *const *ws, 
 hipError_t launch_swiglu_q4k(dwim_dev *dev, const dwim_weight *gate, const dwim_weight *up, float *out, const float *x,
                              size_t n, const float *norm, float eps) {
     if (gate->rows != up->rows || gate->cols != up->cols) return hipErrorInvalidValue;
-    if (n >= kRowsQ4kTokens && n < kGemmTokens) {
+    if (by_rows(n, out, x)) {
         const float *xn = normalized(dev, x, norm, eps, n, gate->cols, nullptr);
         return xn ? launch_rows(dev, gate, up, out, xn, n, 0) : hipErrorOutOfMemory;
     }
-    if (n < kRowsQ4kTokens) {
+    if (!by_gemm(n, out, x)) {
         const dwim_weight *ws[2] = {gate, up};
         float *outs[2] = {out, nullptr};
         return launch_mv_q4k_mfma_tokens(dev, ws, outs, nullptr, 2, 1, x, n, norm, eps, nullptr);

@@ -732,8 +732,9 @@ hipError_t launch_mv_q4k_mfma_tokens(dwim_dev *dev, const dwim_weight *const *ws
         // one token's planes are made in the product's own launch, each wave
         // those of its blocks: 4.7 against 6.1 us for a 1024×1024 matrix, 16.4
         // against 17.5 for 5120×17408, even for a 17408×5120 pair (25.7, 25.9),
-        // each range of whose row is converted for every tile
-        const bool raw = nt == 1 && !norm;
+        // each range of whose row is converted for every tile.  Not in place:
+        // there a workgroup would read what another has written.
+        const bool raw = nt == 1 && !norm && outs[0] != x && (count < 2 || outs[1] != x);
         if (gate_z)
             k_planes_gated<<<dim3(blocks, (unsigned)nt), kPlanesThreads, 0, dev->stream>>>(
                 gate_z + t0 * cols, x + t0 * cols, norm, eps, planes_area(dev, kBatchArea, cols));

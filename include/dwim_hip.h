@@ -117,7 +117,9 @@ int dwim_alloc_cache_f16(dwim_dev *dev, size_t len, dwim_cache **out);
 
 /* ---- operations (gpu/mod.rs:251-400) ---- */
 
-/* Device::matmul (gpu/mod.rs:254): out[t] = w · x[t] for each token row of x. */
+/* Device::matmul (gpu/mod.rs:254): out[t] = w · x[t] for each token row of x.  Here and in the two
+ * operations below the result and the input (x, input) are different buffers, as the reference's
+ * borrows have it; only with Q4_K weights may a product be in place (square ones). */
 int dwim_matmul(dwim_dev *dev, dwim_buf *out, const dwim_weight *w, const dwim_buf *x);
 /* Device::matmul_add (gpu/mod.rs:259-268): x += w · input (scratch as long as x, left undefined). */
 int dwim_matmul_add(dwim_dev *dev, dwim_buf *x, const dwim_weight *w, const dwim_buf *input,

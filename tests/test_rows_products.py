@@ -191,3 +191,36 @@ def test_q4_k_five_to_sixty_four_tokens(gpu, rows, cols, n):
     bound = 1.1 * e * size(wg) * np.abs(b) + np.abs(a) * e * size(wu) + 1.1 * e * e * size(wg) * size(wu) + 2.0 ** -20 * np.abs(want)
     fine = np.arange(n) != n // 2  # (that row's products overflow f32)
     assert (np.abs(got - want) <= bound + 1e-37)[fine].all()
+
+
+@pytest.mark.parametrize("size", [256, 1280, 2560])
+@pytest.mark.parametrize("n", [1, 3, 5, 15, 16, 40, 64, 65])
+def test_q4_k_products_in_place(gpu, size, n):
+    """A square Q4_K product, the add and the pair with the result in the
+    input's own buffer, against the same into another buffer.  Where in-place
+    calls take another kernel the two differ by both kernels' roundings: the
+    bound of a result in the tests above, twice (2^-24 as there, of sums that
+    are at most the row's |w||x| and the blocks' ranges)."""
+    r = np.random.default_rng(size + n)
+    def make():
+        w = O.Weight.quantized(O.Q4_K, (r.normal(0, 0.05, (size, size))).astype(np.float32))
+        return gpu.upload(D.Tensor(D.Q4_K, size, size, w.quants)), w.dequantize().reshape(size, size).astype(np.float64)
+    (g, wg), (u, wu) = make(), make()
+    x = r.normal(0, 1, (n, size)).astype(np.float32)
+    x64, e = np.abs(x.astype(np.float64)), 2 * (64 + size / 16 + 4) * 2.0 ** -24
+    def bound(w):
+        return e * (x64 @ (np.abs(w) + 2 * np.abs(w).max()).T)
+    def both(op):
+        apart, inside, out = gpu.buffer(x.ravel()), gpu.buffer(x.ravel()), gpu.buffer(x.ravel())
+        op(out, apart)
+        op(inside, inside)
+        return gpu.read(out).reshape(n, size).astype(np.float64), gpu.read(inside).reshape(n, size).astype(np.float64)
+    want, got = both(lambda o, i: gpu.matmul(o, g, i))
+    assert (np.abs(got - want) <= bound(wg)).all()
+    scratch = gpu.alloc(n * size)
+    want, got = both(lambda o, i: gpu.matmul_add(o, g, i, scratch))
+    assert (np.abs(got - want) <= bound(wg) + e * x64).all()
+    a, b = np.abs(x.astype(np.float64) @ wg.T), np.abs(x.astype(np.float64) @ wu.T)
+    want, got = both(lambda o, i: gpu.swiglu(o, g, u, i, scratch))
+    # |silu'| <= 1.1 and |silu(g)| <= |g|
+    assert (np.abs(got - want) <= 1.1 * bound(wg) * (b + bound(wu)) + a * bound(wu) + 2.0 ** -20 * np.abs(want)).all()
