@@ -1092,7 +1092,7 @@ struct dwim_model {
         const size_t shapes[][2] = {{q_dim(), H}, {kv_dim(), H}, {H, q_dim()}, {2 * k_dim() + v_dim(), H},
                                     {v_dim(), H}, {H, v_dim()}, {I, H}, {H, I}, {H, H}};
         size_t split = 0, parts = 0, cols_max = 0;
-        if (head->fmt != DWIM_Q4_K) rows_scratch(dev, head->fmt, c.vocab, H, kMaxDrafts + 1, false, &split, &parts);
+        rows_scratch(dev, head->fmt, c.vocab, H, kMaxDrafts + 1, false, &split, &parts);
         const size_t rows_most = fmt == DWIM_Q4_K ? std::min(most, kGemmTokens - 1) : most;
         for (auto &rc : shapes) rows_scratch(dev, fmt, rc[0], rc[1], rows_most, false, &split, &parts);
         rows_scratch(dev, fmt, I, H, rows_most, true, &split, &parts);

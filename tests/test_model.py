@@ -455,3 +455,20 @@ def test_speculative_sampling_with_the_device_sampler(settings):
     if settings[0] == 0.0:
         # at temperature zero sampling is greedy decoding
         assert out == _greedy(M.Model(gpu, cfg, SEED + 2, max_len=96), prompt, 30)
+
+
+@pytest.mark.gpu
+def test_verifying_through_a_q4_k_head_allocates_nothing():
+    """A forward pass finds its scratch reserved, the head's included: 9 tokens
+    through 328704 × 1024 Q4_K rows are 2568 workgroups of 128 rows in two runs
+    of columns (five rounds of 512 and a short one), 24 MB of partial sums."""
+    gpu = D.Hip(0)
+    cfg = M.config_tiny()
+    cfg.vocab = 328704
+    m = M.Model(gpu, cfg, SEED, head_format=D.Q4_K, max_len=64)
+    m.forward(PREFIX, 0)
+    gpu.sync()
+    free = gpu.memory()
+    m.verify([7 * i + 3 for i in range(9)], 5)
+    gpu.sync()
+    assert free - gpu.memory() < 4 << 20
