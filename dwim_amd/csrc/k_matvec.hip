@@ -57,25 +57,27 @@ __global__ void __launch_bounds__(256) k_rows_bf16(const uint16_t *__restrict__ 
 // The most tokens that go through the kernel that converts the activations
 // itself (k_rows_few.hip); more go through the GEMM (k_gemm_rows.hip), whose
 // split of the activations and sum of the parts are launches of their own.
-// Measured on MI355X (us, few | GEMM): a 17408×5120 Q4_0 pair at 16 tokens 44 |
-// 49, at 32 64 | 54, at 64 102 | 76; Q8_0 at 16 53 | 56, at 32 74 | 61; 5120×17408
-// Q4_0 at 16 32 | 50, at 32 46 | 52, at 64 76 | 68; Q6_K, whose GEMM scales every 16
-// columns, at 64 100 | 120; 1024×1024 Q4_0 at 64 12 | 18.
-static size_t few_tokens(const dwim_weight *w) {
-    if (w->fmt == DWIM_Q6_K || w->rows * w->cols <= (size_t)8 << 20) return 64;
-    return w->cols >= 2 * w->rows ? 32 : 16;
+// Measured on MI355X (us, few | GEMM): a 17408×5120 Q4_0 pair at 16 tokens 43 |
+// 44, at 32 66 | 48; Q8_0 at 16 53 | 53, at 32 79 | 57; Q6_K at 16 56 | 72, at 32 93
+// | 76; bf16 at 32 113 | 121, at 64 254 | 139; a 2304×3072 Q8_0 pair at 32 17.5 | 17.8,
+// at 64 32 | 24; 5120×17408 Q4_0 at 16 32 | 47, at 32 44 | 48, at 64 75 | 68; Q6_K,
+// whose GEMM scales every 16 columns, at 64 93 | 116; 1024×1024 Q4_0 at 64 12 | 15.
+static size_t few_tokens(const dwim_weight *w, bool pair) {
+    const bool small = w->rows * w->cols <= (size_t)8 << 20;
+    if (!pair && (small || w->fmt == DWIM_Q6_K)) return 64;
+    return small || w->fmt == DWIM_BF16 || w->cols >= 2 * w->rows ? 32 : 16;
 }
 
 hipError_t launch_rows(dwim_dev *dev, const dwim_weight *w, const dwim_weight *up, float *out, const float *x, size_t n,
                        int add, bool *split) {
-    if (n > few_tokens(w)) {
+    if (n > few_tokens(w, up)) {
         const hipError_t e = launch_gemm_rows(dev, w, up, out, x, n, add, split && *split);
         if (e == hipSuccess && split) *split = true;
         if (e != hipErrorNotSupported) return e;
     }
     // (also a batch whose GEMM cannot have its scratch: the weights read again
     // for every run of tokens)
-    const size_t most = std::min((size_t)64, std::max((size_t)1, ((size_t)1 << 32) / w->cols));
+    const size_t most = std::min((size_t)(up ? 32 : 64), std::max((size_t)1, ((size_t)1 << 32) / w->cols));
     for (size_t t = 0; t < n; t += most) {
         const size_t m = std::min(most, n - t);
         const hipError_t e = launch_rows_few(dev, w, up, out + t * w->rows, x + t * w->cols, m, add);
@@ -91,7 +93,7 @@ void rows_scratch(const dwim_dev *dev, int fmt, size_t rows, size_t cols, size_t
     w.rows = rows;
     w.cols = cols;
     for (size_t n = 1; n <= most; n++) {
-        if (n > few_tokens(&w)) gemm_rows_scratch(dev, fmt, rows, cols, n, pair, split, parts);
+        if (n > few_tokens(&w, pair)) gemm_rows_scratch(dev, fmt, rows, cols, n, pair, split, parts);
         else *parts = std::max(*parts, rows_few_scratch(dev, fmt, rows, cols, n, pair));
     }
 }

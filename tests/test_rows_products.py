@@ -1,12 +1,13 @@
-"""Products in the row-major formats (Q4_0, Q8_0, Q6_K, BF16) on the matrix
-cores, against float64 products of the same dequantized weights, at the sizes
-where their tiles, steps and parts end.
+"""Products on the matrix cores (Q4_0, Q8_0, Q6_K, BF16, and Q4_K) against
+float64 products of the same dequantized weights, at the sizes where their
+tiles, steps and parts end.
 
 The bound: a result is a sum of cols products, each of an exact weight and an
-activation kept to 24 bits (2^-24 of it), summed in f32.  Sums of at most 64
-products round inside a block, then a sum of at most cols/16 block sums: every
-rounding is at most 2^-24 of a partial sum, itself at most Σ|w||x|.  So
-(64 + cols/16 + 4) · 2^-24 · Σ|w||x| holds for any order of summation."""
+activation kept to 23 bits (2^-23 of it: two of the last term's 2^-24), summed
+in f32.  Sums of at most 64 products round inside a block, then a sum of at most
+cols/16 block sums: every rounding is at most 2^-24 of a partial sum, itself at
+most Σ|w||x|.  So (64 + cols/16 + 4) · 2^-24 · Σ|w||x| holds for any order of
+summation."""
 import numpy as np
 import pytest
 
@@ -127,6 +128,43 @@ def test_activations_of_any_size(gpu, name, n):
             assert np.array_equal(got[2], np.where(w[:, 40] == 0, np.nan, -np.inf * w[:, 40]).astype(np.float32), equal_nan=True)
     if n > 3:
         check(got[3:], w, clean[3:])
+
+
+def errors(gpu, name, rows, cols, n, seed):
+    """results less the true ones, over the true ones' root mean square
+    (an add to zeros: Q6_K's plain products of few tokens run on int8 planes)"""
+    t, w = weight(name, rows, cols, seed)
+    x = np.random.default_rng(seed).standard_normal((n, cols), dtype=np.float32)
+    out = gpu.buffer(np.zeros(n * rows, np.float32))
+    gpu.matmul_add(out, gpu.upload(t), gpu.buffer(x), gpu.alloc(n * rows))
+    want = x.astype(np.float64) @ w.T
+    return (gpu.read(out).reshape(n, rows) - want) / np.sqrt((want ** 2).mean())
+
+
+FEW, BATCH = [1, 2, 5, 16], [40, 130]  # tokens through the one kernel and the other
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("n", FEW)
+def test_products_err_up_as_often_as_down(gpu, name, n):
+    """The matrix cores' sums round down.  Unless that is made up for, the mean
+    error over 5120 columns is 4e-8 to 8e-8 of the results' size, where that of
+    unbiased errors of 1.2e-7 over 2048 rows and n tokens is under
+    1.2e-7 / sqrt(2048 n) (here: five times that)."""
+    err = errors(gpu, name, 2048, 5120, n, 11)
+    assert abs(err.mean()) <= 5 * 1.2e-7 / np.sqrt(err.size)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("n", FEW)
+def test_long_rows_round_no_more_than_f32_sums(gpu, name, n):
+    """17408 columns.  A chain of k sums that grow to the result's size has
+    k/2 · u² of error, u = 2^-24 · 0.42 (the mean square of a rounding): 8 block
+    sums a unit, at most 34 units a run of columns, 8 runs, and about 8 inside
+    the blocks, 29 u² = (1.35e-7)².  On the vector ALUs it was 1.3e-7 (bf16 1.4e-7),
+    with every block's sum joining the row's (and rounding down) 1.7e-7 to 2.7e-7."""
+    err = errors(gpu, name, 512, 17408, n, 12)
+    assert np.sqrt((err ** 2).mean()) <= 1.5e-7
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 256), (17, 512), (40, 1280), (64, 1536), (100, 2304), (8200, 1280), (33, 5120), (50, 20480)])
