@@ -94,7 +94,7 @@ def test_swiglu_pair(gpu, name, rows, cols, n):
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
-@pytest.mark.parametrize("n", [1, 2, 4, 5, 16, 40])
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 16, 40, 65, 130])
 def test_activations_of_any_size(gpu, name, n):
     """Rows far beyond f16's range on either side, of zeros, of an outlier
     among tiny values; then infinities and NaN, which stay in their tokens."""
@@ -145,7 +145,7 @@ FEW, BATCH = [1, 2, 5, 16], [40, 130]  # tokens through the one kernel and the o
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
-@pytest.mark.parametrize("n", FEW)
+@pytest.mark.parametrize("n", FEW + BATCH)
 def test_products_err_up_as_often_as_down(gpu, name, n):
     """The matrix cores' sums round down.  Unless that is made up for, the mean
     error over 5120 columns is 4e-8 to 8e-8 of the results' size, where that of
@@ -156,7 +156,7 @@ def test_products_err_up_as_often_as_down(gpu, name, n):
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
-@pytest.mark.parametrize("n", FEW)
+@pytest.mark.parametrize("n", FEW + BATCH)
 def test_long_rows_round_no_more_than_f32_sums(gpu, name, n):
     """17408 columns.  A chain of k sums that grow to the result's size has
     k/2 · u² of error, u = 2^-24 · 0.42 (the mean square of a rounding): 8 block
@@ -165,6 +165,58 @@ def test_long_rows_round_no_more_than_f32_sums(gpu, name, n):
     with every block's sum joining the row's (and rounding down) 1.7e-7 to 2.7e-7."""
     err = errors(gpu, name, 512, 17408, n, 12)
     assert np.sqrt((err ** 2).mean()) <= 1.5e-7
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("n", [1, 20, 65, 130])
+def test_an_outlier_does_not_cost_other_columns_their_bits(gpu, name, n):
+    """A value 1e10 times the others, under weights that are 0 from there to
+    column 512 (as far as an activation's parts may share its scale): the results are the
+    other columns', within the bound of their own sizes."""
+    rows, cols = 70, 2304
+    fmt = FORMATS[name][0]
+    rng = O.Rng(3)
+    if name == "q6_k":
+        vals = (rng.floats(rows * cols) * 0.05).reshape(rows, cols)
+        vals[:, :512] = 0
+        w = O.Weight.quantized(O.Q6_K, vals)
+    else:
+        w = {"q4_0": rng.q4_0, "q8_0": rng.q8_0, "bf16": rng.bf16}[name](rows, cols)
+        (w.quants if name == "bf16" else w.scales).reshape(rows, -1)[:, :512 if name == "bf16" else 16] = 0
+    x = np.random.default_rng(n).standard_normal((n, cols), dtype=np.float32)
+    x[:, 7] = 1e10
+    out = gpu.buffer(np.zeros(n * rows, np.float32))
+    gpu.matmul_add(out, gpu.upload(D.Tensor(fmt, rows, cols, w.quants, w.scales)), gpu.buffer(x), gpu.alloc(n * rows))
+    check(gpu.read(out), w.dequantize().reshape(rows, cols).astype(np.float64), x)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+def test_whole_rounds_of_tiles_and_a_second_launch(gpu, name):
+    """9 × 64 tiles of 4096 tokens, 512 of them whole (two to each of 256 CUs) and 64 in
+    parts, then 33 tokens more in a launch of their own; a product and a pair.
+    5120 columns: at most 32 roundings a run of 512 (Q6_K 16 of 256), 10 (20) of
+    the totals, about 8 inside the blocks: 22 u² = (1.2e-7)² (see above)."""
+    n, cols = 4096 + 33, 5120
+    x = np.random.default_rng(5).standard_normal((n, cols), dtype=np.float32)
+    some = np.unique(np.concatenate([np.arange(0, n, 97), [63, 64, 3583, 3584, 4095, 4096, n - 1]]))
+    gx, xs = gpu.buffer(x), x[some].astype(np.float64)
+    t, w = weight(name, 2304, cols, 6)
+    out = gpu.alloc(n * 2304)
+    gpu.matmul(out, gpu.upload(t), gx)
+    got = gpu.read(out).reshape(n, -1)[some]
+    check(got, w, x[some])
+    want = xs @ w.T
+    assert np.linalg.norm(got - want) <= 1.4e-7 * np.linalg.norm(want)
+    (tg, wg), (tu, wu) = weight(name, 1152, cols, 7), weight(name, 1152, cols, 8)
+    out = gpu.alloc(n * 1152)
+    gpu.swiglu(out, gpu.upload(tg), gpu.upload(tu), gx, gpu.alloc(n * 1152))
+    g, u = xs @ wg.T, xs @ wu.T
+    sg, su = np.abs(xs) @ np.abs(wg).T, np.abs(xs) @ np.abs(wu).T
+    with np.errstate(over="ignore"):
+        want = g / (1 + np.exp(-g)) * u
+    e = (64 + cols / 16 + 4) * 2.0 ** -24
+    bound = 1.1 * e * sg * np.abs(u) + np.abs(g) * e * su + 1.1 * e * e * sg * su + 2.0 ** -20 * np.abs(want) + 1e-37
+    assert (np.abs(gpu.read(out).reshape(n, -1)[some] - want) <= bound).all()
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 256), (17, 512), (40, 1280), (64, 1536), (100, 2304), (8200, 1280), (33, 5120), (50, 20480)])
