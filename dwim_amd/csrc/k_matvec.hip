@@ -1,7 +1,7 @@
 // Matrix products by format and batch size: out[t][r] (+)= w[r] · x[t] (dwim
-// gpu/cpu.rs:110-149, Device::matmul), and the kernel for a
-// few tokens through bf16 matrices of few rows (DeltaNet's gate projection) on
-// the vector ALUs.
+// gpu/cpu.rs:110-149, Device::matmul), and the kernels for a few tokens through
+// bf16 matrices on the vector ALUs: of few rows (DeltaNet's gate projection),
+// and of any.
 #include "device_util.h"
 #include "quant_math.h"
 #include "runtime.h"
@@ -54,6 +54,125 @@ __global__ void __launch_bounds__(256) k_rows_bf16(const uint16_t *__restrict__ 
     }
 }
 
+// Up to four tokens through a bf16 matrix: a group of LPR lanes takes R rows (of
+// each matrix of a SwiGLU pair) and walks their columns 8 at a time, every
+// activation loaded serving its R rows, every weight its T tokens; the lanes' sums
+// meet by lane swaps.  No LDS, no barrier and a wave for every few rows: the
+// weights' way from memory bounds it.  The matrix cores' kernel holds 16 rows a wave and a
+// workgroup for every 16 or 32 rows, too few in flight for weights of two bytes.
+// Measured on MI355X, us, k_rows_few | here, weights from HBM: 5120×5120 1 token
+// 16.8 | 10.4 (5.0 TB/s), 2 18.9 | 11.7, 3 23.2 | 14.9, 4 23.3 | 18.7; 5120×17408
+// 45.8 | 31.3, 53 | 35, 70 | 51, 70 | 61; 17408×5120 42.6 | 33.4, 45 | 40, 54 | 49, 54 |
+// 53; 1000×4096 9.9 | 6.2; 1024×1024 (in the cache) 3.7 | 3.4, 2 4.4 | 3.5; pairs
+// 17408×5120 70 | 61, 75 | 66, 83 | 70, 5120×17408 84 | 64, 91 | 73.  At 5
+// tokens, read twice here, 1000×4096 would be 8.5 | 9.1, larger ones slower than there.
+constexpr int kVecThreads = 256;
+
+template <int R, int T, int LPR, bool PAIR>
+__global__ void __launch_bounds__(kVecThreads) k_vec_bf16(const uint16_t *__restrict__ w, const uint16_t *__restrict__ up,
+                                                          const float *__restrict__ x, float *out, size_t rows,
+                                                          size_t cols, int add) {
+    constexpr int M = PAIR ? 2 : 1;
+    const size_t row0 = ((size_t)blockIdx.x * kVecThreads + threadIdx.x) / LPR * R;
+    const int sl = threadIdx.x & (LPR - 1);
+    if (row0 >= rows) return;  // (whole groups: lane swaps stay within one)
+    const size_t chunks = cols / 8;
+    float acc[M][R][T];
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int t = 0; t < T; t++) acc[m][r][t] = 0.0f;
+    for (size_t c = sl; c < chunks; c += LPR) {
+        // (every load of the step before its sums: left to itself the compiler
+        // waits for each before it issues the next)
+        uint4 q[M][R];
+        float4 xv[T][2];
+#pragma unroll
+        for (int m = 0; m < M; m++)
+#pragma unroll
+            for (int r = 0; r < R; r++) {  // (rows past the last: the last, not written)
+                const size_t row = row0 + r < rows ? row0 + r : rows - 1;
+                q[m][r] = ((const uint4 *)(m ? up : w))[row * chunks + c];
+            }
+#pragma unroll
+        for (int t = 0; t < T; t++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) xv[t][i] = ((const float4 *)(x + t * cols))[2 * c + i];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < M; m++)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int t = 0; t < T; t++) {
+                    const uint4 v = q[m][r];
+                    const float4 a = xv[t][0], b = xv[t][1];
+                    auto lo = [](uint32_t u) { return __uint_as_float(u << 16); };
+                    auto hi = [](uint32_t u) { return __uint_as_float(u & 0xffff0000u); };
+                    float sum = fmaf(hi(v.x), a.y, lo(v.x) * a.x);  // (by itself: see k_rows_few.hip)
+                    sum = fmaf(hi(v.y), a.w, fmaf(lo(v.y), a.z, sum));
+                    sum = fmaf(hi(v.z), b.y, fmaf(lo(v.z), b.x, sum));
+                    acc[m][r][t] += fmaf(hi(v.w), b.w, fmaf(lo(v.w), b.z, sum));
+                }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            const float v = group_sum<LPR>(acc[0][r][t]), u = PAIR ? group_sum<LPR>(acc[M - 1][r][t]) : 0.0f;
+            if (sl == 0 && row0 + r < rows) {
+                float *o = out + t * rows + row0 + r;
+                *o = PAIR ? v * sigmoidf_(v) * u : add ? *o + v : v;
+            }
+        }
+}
+
+template <int R, int T, bool PAIR>
+static hipError_t vec_bf16(hipStream_t s, const dwim_weight *w, const dwim_weight *up, float *out, const float *x, int add) {
+    // lanes a group: all 64, whose loads are whole lines, unless a fifth of their
+    // steps would be past the row's end
+    const size_t chunks = w->cols / 8;
+    int lpr = 64;
+    for (int l = 32; l >= 4; l >>= 1)
+        if ((chunks + l - 1) / l * l * 5 < (chunks + lpr - 1) / lpr * lpr * 4) lpr = l;
+    const unsigned blocks = (unsigned)(((w->rows + R - 1) / R * lpr + kVecThreads - 1) / kVecThreads);
+    const uint16_t *q = (const uint16_t *)w->q, *u = up ? (const uint16_t *)up->q : nullptr;
+    switch (lpr) {
+    case 64: k_vec_bf16<R, T, 64, PAIR><<<blocks, kVecThreads, 0, s>>>(q, u, x, out, w->rows, w->cols, add); break;
+    case 32: k_vec_bf16<R, T, 32, PAIR><<<blocks, kVecThreads, 0, s>>>(q, u, x, out, w->rows, w->cols, add); break;
+    case 16: k_vec_bf16<R, T, 16, PAIR><<<blocks, kVecThreads, 0, s>>>(q, u, x, out, w->rows, w->cols, add); break;
+    case 8: k_vec_bf16<R, T, 8, PAIR><<<blocks, kVecThreads, 0, s>>>(q, u, x, out, w->rows, w->cols, add); break;
+    default: k_vec_bf16<R, T, 4, PAIR><<<blocks, kVecThreads, 0, s>>>(q, u, x, out, w->rows, w->cols, add); break;
+    }
+    return hipGetLastError();
+}
+
+// Tokens that go there.
+constexpr size_t kVecTokens = 4;
+
+// Rows a group: where rows are many, more of them share the activations (17408
+// rows, one token: 1 row a group 36, 4 33; at 5120 rows 4 took 11.8 for 10.4)
+template <int T>
+static hipError_t vec_bf16_tokens(hipStream_t s, const dwim_weight *w, const dwim_weight *up, float *out, const float *x,
+                                  int add) {
+    constexpr int kFew = T == 1 ? 1 : 2, kMany = T == 1 ? 4 : 2;
+    const bool many = w->rows >= 16384;
+    if (up) return many ? vec_bf16<2, T, true>(s, w, up, out, x, 0) : vec_bf16<1, T, true>(s, w, up, out, x, 0);
+    return many ? vec_bf16<kMany, T, false>(s, w, up, out, x, add) : vec_bf16<kFew, T, false>(s, w, up, out, x, add);
+}
+
+static hipError_t launch_vec_bf16(hipStream_t s, const dwim_weight *w, const dwim_weight *up, float *out, const float *x,
+                                  size_t n, int add) {
+    switch (n) {
+    case 1: return vec_bf16_tokens<1>(s, w, up, out, x, add);
+    case 2: return vec_bf16_tokens<2>(s, w, up, out, x, add);
+    case 3: return vec_bf16_tokens<3>(s, w, up, out, x, add);
+    default: return vec_bf16_tokens<4>(s, w, up, out, x, add);
+    }
+}
+
 // The most tokens that go through the kernel that converts the activations
 // itself (k_rows_few.hip); more go through the GEMM (k_gemm_rows.hip), whose
 // split of the activations and sum of the parts are launches of their own.
@@ -70,6 +189,7 @@ static size_t few_tokens(const dwim_weight *w, bool pair) {
 
 hipError_t launch_rows(dwim_dev *dev, const dwim_weight *w, const dwim_weight *up, float *out, const float *x, size_t n,
                        int add, bool *split) {
+    if (up && (up->fmt != w->fmt || up->rows != w->rows || up->cols != w->cols)) return hipErrorInvalidValue;
     if (n > few_tokens(w, up)) {
         const hipError_t e = launch_gemm_rows(dev, w, up, out, x, n, add, split && *split);
         if (e == hipSuccess && split) *split = true;
@@ -80,7 +200,10 @@ hipError_t launch_rows(dwim_dev *dev, const dwim_weight *w, const dwim_weight *u
     const size_t most = std::min((size_t)(up ? 32 : 64), std::max((size_t)1, ((size_t)1 << 32) / w->cols));
     for (size_t t = 0; t < n; t += most) {
         const size_t m = std::min(most, n - t);
-        const hipError_t e = launch_rows_few(dev, w, up, out + t * w->rows, x + t * w->cols, m, add);
+        float *const o = out + t * w->rows;
+        const float *const xt = x + t * w->cols;
+        const hipError_t e = w->fmt == DWIM_BF16 && m <= kVecTokens ? launch_vec_bf16(dev->stream, w, up, o, xt, m, add)
+                                                                     : launch_rows_few(dev, w, up, o, xt, m, add);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

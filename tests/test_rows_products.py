@@ -93,6 +93,26 @@ def test_swiglu_pair(gpu, name, rows, cols, n):
     assert (np.abs(gpu.read(out).reshape(n, rows) - want) <= bound).all()
 
 
+@pytest.mark.parametrize("rows,cols", [(16383, 24), (16384, 520), (16387, 40)])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5])
+def test_bf16_of_many_rows(gpu, rows, cols, n):
+    """The vector kernel's rows a group (1, 2 and 4) and lanes a group (4, 8 and
+    64) where they change, and 5 tokens past it; an add and a pair."""
+    (t, w), (tu, wu) = weight("bf16", rows, cols, 3), weight("bf16", rows, cols, 4)
+    x = O.Rng(n).floats(n * cols).reshape(n, cols)
+    base = O.Rng(n + 1).floats(n * rows)
+    gw, gx, acc, out = gpu.upload(t), gpu.buffer(x), gpu.buffer(base), gpu.alloc(n * rows)
+    gpu.matmul_add(acc, gw, gx, gpu.alloc(n * rows))
+    check(gpu.read(acc), w, x, base.reshape(n, rows).astype(np.float64))
+    gpu.swiglu(out, gw, gpu.upload(tu), gx, gpu.alloc(n * rows))
+    g, u = x.astype(np.float64) @ w.T, x.astype(np.float64) @ wu.T
+    sg, su = np.abs(x) @ np.abs(w).T, np.abs(x) @ np.abs(wu).T
+    e = (64 + cols / 16 + 4) * 2.0 ** -24
+    want = g / (1 + np.exp(-g)) * u
+    bound = 1.1 * e * sg * np.abs(u) + np.abs(g) * e * su + 1.1 * e * e * sg * su + 2.0 ** -20 * np.abs(want) + 1e-37
+    assert (np.abs(gpu.read(out).reshape(n, rows) - want) <= bound).all()
+
+
 @pytest.mark.parametrize("name", list(FORMATS))
 @pytest.mark.parametrize("n", [1, 2, 4, 5, 16, 40, 65, 130])
 def test_activations_of_any_size(gpu, name, n):
