@@ -37,6 +37,7 @@ typedef _Float16 ahalf8 __attribute__((ext_vector_type(8)));
 typedef float afloat4 __attribute__((ext_vector_type(4)));
 
 constexpr int kFD = 256, kFQ = 128, kFThreads = 256;
+constexpr size_t kMPerCU = 2;  // blocks of k_attn_mfma resident at once on a CU (its launch bounds)
 constexpr size_t kFlashItems = 2;  // blocks a CU when a batch's positions are split
 
 
@@ -271,7 +272,8 @@ __global__ void __launch_bounds__(kPThreads) k_attn_partial(float *__restrict__ 
 // values on the f16 matrix cores (v_mfma_f32_16x16x32_f16).  A block of 4
 // waves takes a run of sh.ch positions (64 a step) of one key/value head and
 // its query rows, a row a (token, head) pair: the G heads of one token, or
-// of up to kTok tokens of a small batch, in RT tiles of 16 rows.
+// of up to kTok tokens of a small batch, in RT tiles of 16 rows.  (The queries
+// are staged times qscale, a power of two.)
 //   * Scores, wave w the step's positions 16w..16w+15: for each Q8 block of
 //     32 dimensions, the queries' f16 hi and lo parts (staged in LDS once) as
 //     A against the keys as B, exact in f16 (int8, or the f16 cache as is),
@@ -316,7 +318,8 @@ __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ 
                                                          const int8_t *__restrict__ kq,
                                                          const uint16_t *__restrict__ ks,
                                                          const int8_t *__restrict__ vq,
-                                                         const uint16_t *__restrict__ vs, Shape sh, int G, int T) {
+                                                         const uint16_t *__restrict__ vs, Shape sh, int G, int T,
+                                                         float qscale) {
     constexpr int NR = 16 * RT;  // rows, padded
     constexpr int D = kFD;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
@@ -346,7 +349,7 @@ __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ 
     for (int r = wave; r < NR; r += kMThreads / 64) {
         float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (r < R) x = *(const float4 *)(q + ((t0 + r / G) * sh.n_heads + head0 + r % G) * D + 4 * lane);
-        const float xs[4] = {x.x, x.y, x.z, x.w};
+        const float xs[4] = {x.x * qscale, x.y * qscale, x.z * qscale, x.w * qscale};
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const _Float16 h = (_Float16)xs[e];
@@ -363,7 +366,7 @@ __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ 
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
         for (int j = 0; j < 4; j++) o[rt][j] = afloat4{0.0f, 0.0f, 0.0f, 0.0f};
-    const float scale = 1.0f / 16.0f;  // 1 / sqrt(256)
+    const float scale = 0.0625f / qscale;  // 1 / sqrt(256), powers of two
     const int steps = (int)(sh.ch / kMStep);
     // ---- loads: this wave's keys (position 16w + r16, 8 dimensions of each
     // Q8 block) and their scales; a 4-dimension x 16-position patch of the
@@ -1066,6 +1069,26 @@ unsigned flash_parts(const dwim_dev *dev, size_t n, size_t pos, size_t n_heads, 
     }
     return (unsigned)best;
 }
+
+// Tokens a block where a batch of few rows over few positions goes to the
+// decode pass (k_attn_mfma), 0 where not: as long as that pass's blocks are all resident at
+// once.  There is no cache to expand then, and none of what a block of
+// k_attn_flash does once (its queries, a prologue of two steps, the scores of
+// the step past the last), most of its time when the steps are few.  Measured on
+// MI355X (us, flash | so), 24 / 4 heads, q8: 16 tokens at position 0 16.4 | 12, at
+// 100 23 | 13, at 1000 35 | 22, at 4000 (past the blocks' limit) 40 | 36; 32 at 0 17.6 | 16, at
+// 200 32 | 18.  The pass takes 0.2 us more a token (its merge): 64 at 0 20 | 24,
+// hence the limit of rows.
+constexpr size_t kShortRows = 768;
+size_t short_batch_tokens(const dwim_dev *dev, size_t n, size_t pos, size_t n_heads, size_t n_kv_heads) {
+    const size_t G = n_heads / n_kv_heads, slots = kMPerCU * (size_t)dev->cus;
+    const size_t base = (pos + n + kMStep - 1) / kMStep * n_kv_heads;
+    if (n * n_heads > kShortRows) return 0;
+    // (one tile of 16 rows a block, else two: 16 tokens of 24 / 4 heads 12 | 16 us)
+    for (size_t T : {std::min((size_t)kTok, 16 / G), (size_t)kTok})
+        if (base * ((n + T - 1) / T) <= slots) return T;
+    return 0;
+}
 }  // namespace
 
 // The partial results of a batch's positions split over blocks, for any
@@ -1088,8 +1111,6 @@ hipError_t attention_reserve(dwim_dev *dev, size_t floats) {
 
 namespace {
 
-// the matrix-core pass's blocks resident at once on a CU (its launch bounds)
-constexpr size_t kMPerCU = 2;
 // one token over at most this many positions: the one-chunk VALU pass, a
 // single round of blocks (4k positions: 14.1 against 14.2 us with the merge;
 // 32k: 47.8 against 31.2)
@@ -1097,13 +1118,13 @@ constexpr size_t kValuLen = 6144;
 
 template <int RT, bool F16>
 hipError_t mfma_pass(dwim_dev *dev, dim3 grid, float *partials, const float *q, const dwim_cache *k,
-                     const dwim_cache *v, const Shape &sh, int G, int T) {
+                     const dwim_cache *v, const Shape &sh, int G, int T, float qscale) {
     constexpr size_t lds = mfma_lds(RT, F16);
     // once a process (thread-safe: a function-local static)
     static const hipError_t raised =
         hipFuncSetAttribute((const void *)k_attn_mfma<RT, F16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (raised != hipSuccess) return raised;
-    k_attn_mfma<RT, F16><<<grid, kMThreads, lds, dev->stream>>>(partials, q, k->q, k->s, v->q, v->s, sh, G, T);
+    k_attn_mfma<RT, F16><<<grid, kMThreads, lds, dev->stream>>>(partials, q, k->q, k->s, v->q, v->s, sh, G, T, qscale);
     return hipGetLastError();
 }
 
@@ -1124,7 +1145,9 @@ hipError_t flash_pass(dwim_dev *dev, const FlashArgs &fa) {
 hipError_t attention_run(dwim_dev *dev, float *partials, float *out, const float *q, const dwim_cache *k,
                          const dwim_cache *v, size_t n, size_t pos, size_t n_heads, size_t head_dim,
                          size_t n_kv_heads, const float *gate, planes::View pv, uint8_t *kvx, size_t room) {
-    if (n >= 16 && !pv.q && head_dim == (size_t)kFD && n_heads % n_kv_heads == 0) {
+    const size_t few = n >= 16 && !pv.q && head_dim == (size_t)kFD ? short_batch_tokens(dev, n, pos, n_heads, n_kv_heads) : 0;
+    const bool fits = partials && n * n_heads * ((pos + n + kMStep - 1) / kMStep) * (kFD + 2) <= room;
+    if (n >= 16 && !pv.q && head_dim == (size_t)kFD && n_heads % n_kv_heads == 0 && !(few && fits)) {
         // a batch of tokens over the expanded cache (kvx: attention_kvx_bytes)
         const size_t len = pos + n, steps = (len + kXStep - 1) / kXStep;
         dim3 gx((unsigned)steps, (unsigned)n_kv_heads);
@@ -1155,16 +1178,17 @@ hipError_t attention_run(dwim_dev *dev, float *partials, float *out, const float
         // few blocks costs a whole block's time (32k + 1 positions: 412 blocks
         // of 5 steps, not 516 of 4; in the model 43.3 against 47.5 us a
         // 4-token pass, 9.4 against 10.9 us its merge)
-        const int G = (int)(n_heads / n_kv_heads), T = n > 1 ? kTok : 1;
+        const int G = (int)(n_heads / n_kv_heads), T = few ? (int)few : n > 1 ? kTok : 1;
+        const float qscale = few ? 0.0625f : 1.0f;  // (a batch's queries have the range k_attn_flash gives them)
         const size_t groups = (n + T - 1) / T, base = (len + kMStep - 1) / kMStep * n_kv_heads * groups;
         const size_t slots = kMPerCU * (size_t)dev->cus;
         const size_t ch = kMStep * std::max<size_t>(1, (base + slots - 1) / slots), chunks = (len + ch - 1) / ch;
         Shape sh{n, pos, n_heads, head_dim, n_kv_heads, ch, chunks};
         dim3 g1((unsigned)chunks, (unsigned)n_kv_heads, (unsigned)groups);
-        hipError_t e = T * G <= 16 ? (k->f16 ? mfma_pass<1, true>(dev, g1, partials, q, k, v, sh, G, T)
-                                             : mfma_pass<1, false>(dev, g1, partials, q, k, v, sh, G, T))
-                                   : (k->f16 ? mfma_pass<2, true>(dev, g1, partials, q, k, v, sh, G, T)
-                                             : mfma_pass<2, false>(dev, g1, partials, q, k, v, sh, G, T));
+        hipError_t e = T * G <= 16 ? (k->f16 ? mfma_pass<1, true>(dev, g1, partials, q, k, v, sh, G, T, qscale)
+                                             : mfma_pass<1, false>(dev, g1, partials, q, k, v, sh, G, T, qscale))
+                                   : (k->f16 ? mfma_pass<2, true>(dev, g1, partials, q, k, v, sh, G, T, qscale)
+                                             : mfma_pass<2, false>(dev, g1, partials, q, k, v, sh, G, T, qscale));
         if (e != hipSuccess) return e;
         dim3 g2((unsigned)n_heads * (unsigned)(head_dim / 64), (unsigned)n);
         k_attn_combine<<<g2, kCThreads, 0, dev->stream>>>(out, partials, sh, gate, pv);

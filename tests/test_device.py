@@ -689,6 +689,10 @@ def test_argmax_takes_the_first_maximum(gpu):
     (6, 2, 16, 0, False), (6, 2, 16, 16, True), (8, 1, 17, 15, False),      # one step of 32 positions, two
     (6, 2, 16, 2000, False), (4, 2, 33, 3000, True), (24, 4, 40, 977, False),  # positions split over blocks
     (5, 5, 100, 700, True), (24, 4, 300, 100, False), (6, 1, 22, 9, False),
+    (32, 4, 32, 0, False), (32, 4, 25, 8, True), (24, 4, 33, 0, False),     # past the short batches' rows: one step, two
+    (24, 4, 32, 0, True), (24, 4, 16, 48, False), (24, 4, 17, 48, True),    # short batches: one chunk of 64, two
+    (5, 1, 18, 500, False), (3, 1, 17, 63, True), (1, 1, 19, 1, False),     # 3, 4 and 4 tokens a block
+    (24, 4, 16, 1008, False), (24, 4, 16, 1009, True), (24, 4, 16, 2032, True), (24, 4, 16, 2033, False),  # 2 tokens a block, 4, not short (256 CUs)
 ])
 def test_attention_batch_edges_against_float64(gpu, heads, kv, n, pos, f16):
     """The batch kernel at the edges of its tiles, steps and splits.  The cache
