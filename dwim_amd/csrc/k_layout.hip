@@ -59,19 +59,21 @@ unsigned blocks_of(size_t count) { return (unsigned)((count + 255) / 256); }
 
 }  // namespace
 
-hipError_t launch_tile_q4_0(hipStream_t s, void *q, void *scales, const void *src_q, const void *src_s, size_t rows,
-                            size_t cols) {
-    const size_t n = rowt::chunks(rows, cols, 4), m = rowt::scales(rows, cols);
-    k_tile_chunks<<<blocks_of(n), 256, 0, s>>>((uint4 *)q, (const uint4 *)src_q, rows, cols, 4, n);
-    k_tile_scales<<<blocks_of(m), 256, 0, s>>>((uint16_t *)scales, (const uint16_t *)src_s, rows, cols, m);
+hipError_t launch_tile_q4_0(hipStream_t s, void *q, const void *src, size_t rows, size_t cols) {
+    const size_t n = rowt::chunks(rows, cols, 4);
+    k_tile_chunks<<<blocks_of(n), 256, 0, s>>>((uint4 *)q, (const uint4 *)src, rows, cols, 4, n);
     return hipGetLastError();
 }
 
-hipError_t launch_tile_q8_0(hipStream_t s, void *q, void *scales, const void *src_q, const void *src_s, size_t rows,
-                            size_t cols) {
-    const size_t n = rowt::chunks(rows, cols, 8), m = rowt::scales(rows, cols);
-    k_tile_chunks<<<blocks_of(n), 256, 0, s>>>((uint4 *)q, (const uint4 *)src_q, rows, cols, 8, n);
-    k_tile_scales<<<blocks_of(m), 256, 0, s>>>((uint16_t *)scales, (const uint16_t *)src_s, rows, cols, m);
+hipError_t launch_tile_q8_0(hipStream_t s, void *q, const void *src, size_t rows, size_t cols) {
+    const size_t n = rowt::chunks(rows, cols, 8);
+    k_tile_chunks<<<blocks_of(n), 256, 0, s>>>((uint4 *)q, (const uint4 *)src, rows, cols, 8, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_tile_scales(hipStream_t s, void *scales, const void *src, size_t rows, size_t cols) {
+    const size_t n = rowt::scales(rows, cols);
+    k_tile_scales<<<blocks_of(n), 256, 0, s>>>((uint16_t *)scales, (const uint16_t *)src, rows, cols, n);
     return hipGetLastError();
 }
 

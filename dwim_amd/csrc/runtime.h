@@ -285,10 +285,9 @@ hipError_t launch_argmax(hipStream_t s, const float *logits, size_t rows, size_t
 hipError_t launch_synthetic_q4_k(hipStream_t s, uint8_t *tiled, size_t rows, size_t cols,
                                  uint64_t seed, float c);
 // the host formats as copied to the device, into the layouts above (k_layout.hip)
-hipError_t launch_tile_q4_0(hipStream_t s, void *q, void *scales, const void *src_q, const void *src_s, size_t rows,
-                            size_t cols);
-hipError_t launch_tile_q8_0(hipStream_t s, void *q, void *scales, const void *src_q, const void *src_s, size_t rows,
-                            size_t cols);
+hipError_t launch_tile_q4_0(hipStream_t s, void *q, const void *src, size_t rows, size_t cols);
+hipError_t launch_tile_q8_0(hipStream_t s, void *q, const void *src, size_t rows, size_t cols);
+hipError_t launch_tile_scales(hipStream_t s, void *scales, const void *src, size_t rows, size_t cols);  // of either
 hipError_t launch_tile_q6_k(hipStream_t s, void *ql, void *qh, void *sc, void *d, const void *src, size_t rows,
                             size_t cols);
 hipError_t launch_synthetic_q6_k(hipStream_t s, uint8_t *ql, uint8_t *qh, int8_t *sc,

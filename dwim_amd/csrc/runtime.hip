@@ -349,6 +349,26 @@ static int alloc_q6k(dwim_dev *dev, dwim_weight *w) {
            alloc_copy(dev, &w->s2, nullptr, blocks * 16) || alloc_copy(dev, &w->s3, nullptr, blocks * 2);
 }
 
+// `rows` rows of the host's bytes in runs that are copied to a buffer on the device
+// and laid out from there by tile(first row, rows, the copy); whole tiles of
+// rows, of about kSlab bytes (not a second copy of the matrix)
+constexpr size_t kSlab = (size_t)64 << 20;
+template <class Tile>
+static int upload_slabs(dwim_dev *dev, const void *src, size_t rows, size_t row_bytes, Tile tile) {
+    const size_t most = std::max(rowt::kTile, kSlab / row_bytes / rowt::kTile * rowt::kTile);
+    void *raw = nullptr;
+    int err = alloc_copy(dev, &raw, nullptr, std::min(rows, most) * row_bytes);
+    for (size_t r = 0; r < rows && !err; r += most) {
+        const size_t m = std::min(most, rows - r);
+        hipError_t e = hipMemcpyAsync(raw, (const uint8_t *)src + r * row_bytes, m * row_bytes, hipMemcpyHostToDevice, dev->stream);
+        if (e == hipSuccess) e = tile(r, m, raw);
+        if (e != hipSuccess) err = dwim_fail(std::string("uploading a weight: ") + hipGetErrorString(e));
+    }
+    if (hipStreamSynchronize(dev->stream) != hipSuccess && !err) err = dwim_fail("uploading a weight failed");
+    if (raw) (void)hipFree(raw);
+    return err;
+}
+
 static int check_shape(int fmt, size_t rows, size_t cols) {
     DWIM_CHECK(rows > 0 && cols > 0, "an empty weight matrix");
     switch (fmt) {
@@ -374,18 +394,20 @@ extern "C" int dwim_upload(dwim_dev *dev, int fmt, size_t rows, size_t cols, con
     dev->refs++;
     int err = 0;
     size_t nb = cols / 256;
-    void *raw = nullptr, *raw_s = nullptr;  // the host format, to be laid out anew
     switch (fmt) {
     case DWIM_BF16: err = alloc_copy(dev, &w->q, quants, rows * cols * 2); break;
     case DWIM_Q4_0:
     case DWIM_Q8_0: {
-        const size_t per = fmt == DWIM_Q4_0 ? 4 : 8, blocks = rows * cols / 32;
-        err = alloc_copy(dev, &raw, quants, blocks * per * 4) || alloc_copy(dev, &raw_s, scales, blocks * 2) ||
-              alloc_copy(dev, &w->q, nullptr, rowt::chunks(rows, cols, per) * 16) ||
-              alloc_copy(dev, &w->s, nullptr, rowt::scales(rows, cols) * 2);
-        if (!err)
-            err = (fmt == DWIM_Q4_0 ? launch_tile_q4_0 : launch_tile_q8_0)(dev->stream, w->q, w->s, raw, raw_s, rows,
-                                                                           cols) != hipSuccess;
+        const size_t per = fmt == DWIM_Q4_0 ? 4 : 8;
+        err = alloc_copy(dev, &w->q, nullptr, rowt::chunks(rows, cols, per) * 16) ||
+              alloc_copy(dev, &w->s, nullptr, rowt::scales(rows, cols) * 2) ||
+              upload_slabs(dev, quants, rows, cols / 32 * per * 4, [&](size_t r, size_t m, const void *raw) {
+                  uint8_t *q = (uint8_t *)w->q + rowt::chunks(r, cols, per) * 16;
+                  return (fmt == DWIM_Q4_0 ? launch_tile_q4_0 : launch_tile_q8_0)(dev->stream, q, raw, m, cols);
+              }) ||
+              upload_slabs(dev, scales, rows, cols / 32 * 2, [&](size_t r, size_t m, const void *raw) {
+                  return launch_tile_scales(dev->stream, (uint16_t *)w->s + rowt::scales(r, cols), raw, m, cols);
+              });
         break;
     }
     case DWIM_Q4_K: {
@@ -399,14 +421,14 @@ extern "C" int dwim_upload(dwim_dev *dev, int fmt, size_t rows, size_t cols, con
         break;
     }
     case DWIM_Q6_K:
-        err = alloc_copy(dev, &raw, quants, rows * nb * 210) || alloc_q6k(dev, w);
-        if (!err) err = launch_tile_q6_k(dev->stream, w->q, w->s, w->s2, w->s3, raw, rows, cols) != hipSuccess;
+        err = alloc_q6k(dev, w) || upload_slabs(dev, quants, rows, nb * 210, [&](size_t r, size_t m, const void *raw) {
+                  const size_t b = r * nb;
+                  return launch_tile_q6_k(dev->stream, (uint8_t *)w->q + b * 128, (uint8_t *)w->s + b * 64,
+                                          (uint8_t *)w->s2 + b * 16, (uint8_t *)w->s3 + b * 2, raw, m, cols);
+              });
         break;
     }
     if (!err && hipStreamSynchronize(dev->stream) != hipSuccess) err = dwim_fail("uploading a weight failed");
-    if (err && (raw || raw_s)) (void)hipStreamSynchronize(dev->stream);  // whatever still reads the copies
-    if (raw) (void)hipFree(raw);
-    if (raw_s) (void)hipFree(raw_s);
     if (err) {
         dwim_free_weight(w);
         return 1;

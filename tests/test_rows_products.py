@@ -363,3 +363,29 @@ def test_q4_k_long_rows_in_whole_tiles(gpu):
     runs of 16 blocks N/4 · u², 6.0e-7; the line lies between."""
     err = q4_k_errors(gpu, 2048, 8192, 4096, 22, slice(0, 4096, 61))
     assert np.sqrt((err ** 2).mean()) <= 7e-7
+
+
+@pytest.mark.parametrize("name,cols", [("q8_0", 4096), ("q4_0", 8160), ("q6_k", 5120)])
+def test_uploads_of_more_than_a_slab(gpu, name, cols):
+    """A matrix goes to the device 64 MB at a time: the rows at the ends of a
+    slab, read back, and those of the last tile."""
+    fmt = FORMATS[name][0]
+    row_bytes = {"q8_0": cols, "q4_0": cols // 2, "q6_k": cols // 256 * 210}[name]
+    slab = (64 << 20) // row_bytes // 16 * 16
+    rows = slab + 17
+    rng = np.random.default_rng(1)
+    if name == "q6_k":
+        blocks = rng.integers(0, 256, (rows, cols // 256, 210), dtype=np.uint8)
+        blocks[..., 208:] = np.frombuffer(np.float16(0.01).tobytes(), np.uint8)
+        quants, scales = blocks.ravel(), None
+    else:
+        quants = rng.integers(0, 256, rows * row_bytes, dtype=np.uint8)
+        quants = quants.view(np.int8) if name == "q8_0" else quants
+        scales = rng.uniform(0.001, 0.01, rows * cols // 32).astype(np.float16).view(np.uint16)
+    gw = gpu.upload(D.Tensor(fmt, rows, cols, quants, scales))
+    for r in (0, 15, 16, slab - 1, slab, slab + 15, slab + 16):
+        out = gpu.alloc(cols)
+        gpu.embed(out, gw, [r])
+        one = slice(r * row_bytes, (r + 1) * row_bytes), slice(r * (cols // 32), (r + 1) * (cols // 32))
+        want = O.Weight(OFMT[fmt], 1, cols, quants[one[0]], None if scales is None else scales[one[1]]).dequantize()
+        assert np.array_equal(gpu.read(out), np.asarray(want, np.float32).ravel()), r
