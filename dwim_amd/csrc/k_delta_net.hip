@@ -20,6 +20,8 @@
 #include "planes.h"
 #include "runtime.h"
 
+#include <algorithm>
+
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 namespace {
@@ -436,6 +438,7 @@ struct Chunks {
     float *KT;   // [n_k][chunks]: tiles of (keys, tokens): key r, tokens 4kq..
     float *Q;    // [n_k][chunks]: tiles of (tokens, keys): token r, keys 4kq..
 };
+constexpr size_t kRunTokens = 4096;  // tokens a pair of launches: 320 MB of the matrices at 16/48 heads
 constexpr size_t kWide = (size_t)kC * kD, kSquare = (size_t)kC * kC;  // floats of a chunk's matrices
 
 __host__ Chunks chunks_of(float *work, size_t nch, size_t n_k, size_t n_v) {
@@ -651,8 +654,7 @@ __global__ void __launch_bounds__(256, 3) k_dn_prep(const float *__restrict__ q,
 // accumulators hold them (lane (kq, r): rows 4kq.. of column r, 16 bytes), which
 // is also how its B operand takes them.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) k_dn_chunks(
-    float *__restrict__ out, const float *__restrict__ q, const Chunks in, float *__restrict__ state, size_t n, int n_k,
-    int n_v) {
+    float *__restrict__ out, const Chunks in, float *__restrict__ state, size_t n, int n_k, int n_v) {
     __shared__ v4f Ss[8][4][16], Us[4][4][16], Ud[4][4][16];  // [16 rows][kq][column]
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, kq = lane >> 4;
     const int ratio = n_v / n_k;
@@ -816,7 +818,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 // The chunked form's per-chunk matrices (W, Ũ, M, the decays and Kᵀ) for n tokens.
 size_t delta_net_work_floats(size_t n, size_t n_k_heads, size_t n_v_heads) {
     if (n < (size_t)kC) return 0;
-    const size_t nch = (n + kC - 1) / kC;
+    const size_t nch = (std::min(n, kRunTokens) + kC - 1) / kC;
     return nch * (n_v_heads * (2 * kWide + kSquare + 2 * kC) + n_k_heads * 2 * kWide);
 }
 
@@ -848,14 +850,16 @@ hipError_t launch_delta_net(dwim_dev *dev, float *out, const float *q, const flo
     if (head_dim != (size_t)kD || n_k_heads == 0 || n_v_heads % n_k_heads) return hipErrorInvalidValue;
     if (unit_keys && n >= (size_t)kC && !(rms && rms->ss)) {
         if (state_in && state_in != state) return hipErrorInvalidValue;  // (the token loop reads one state, writes another)
-        const size_t nch = (n + kC - 1) / kC;
         hipError_t e = delta_net_reserve(dev, n, n_k_heads, n_v_heads);
         if (e != hipSuccess) return e;
-        const Chunks c = chunks_of(dev->dn_work, nch, n_k_heads, n_v_heads);
-        k_dn_prep<<<dim3((unsigned)nch, (unsigned)n_v_heads), 256, 0, dev->stream>>>(q, k, v, gates, decay, c, n,
-                                                                                   (int)n_k_heads, (int)n_v_heads);
-        k_dn_chunks<<<(unsigned)(8 * n_v_heads), 256, 0, dev->stream>>>(out, q, c, state, n, (int)n_k_heads,
-                                                                         (int)n_v_heads);
+        const int nk = (int)n_k_heads, nv = (int)n_v_heads;
+        for (size_t t = 0; t < n; t += kRunTokens) {
+            const size_t m = std::min(kRunTokens, n - t), nch = (m + kC - 1) / kC, kt = t * n_k_heads * kD, vt = t * n_v_heads * kD;
+            const Chunks c = chunks_of(dev->dn_work, nch, n_k_heads, n_v_heads);
+            k_dn_prep<<<dim3((unsigned)nch, (unsigned)n_v_heads), 256, 0, dev->stream>>>(
+                q + kt, k + kt, v + vt, gates + t * 2 * n_v_heads, decay, c, m, nk, nv);
+            k_dn_chunks<<<(unsigned)(8 * n_v_heads), 256, 0, dev->stream>>>(out + vt, c, state, m, nk, nv);
+        }
         return hipGetLastError();
     }
     dim3 grid(kD / kCols, (unsigned)n_v_heads);

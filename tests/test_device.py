@@ -302,9 +302,9 @@ def test_q4_k_swiglu_and_matmul_add_match_cpu(gpu):
 
 
 def test_q4_k_small_batches_on_the_matrix_cores(gpu):
-    # 2..15 tokens run on the int8 matrix cores in launches of up to four
-    # tokens (7 = 4 + 3, 13 = 4 + 3 + 3 + 3); the 17408 columns split each
-    # tile's blocks over several workgroups
+    # 2..4 tokens run on the int8 matrix cores in one launch, 5 and more through
+    # the kernels of the other formats; the 17408 columns split each tile's
+    # blocks over several workgroups
     for rows, cols, ns in [(1100, 5120, (2, 3, 4, 5, 7, 13)), (300, 17408, (4, 6, 15)), (64, 256, (3,))]:
         w = _k_quantized(O.Q4_K, rows)(rows, cols)
         gw = gpu.upload(to_tensor(w))
@@ -323,11 +323,13 @@ def test_q4_k_small_batches_on_the_matrix_cores(gpu):
     # a SwiGLU pair (two matrices a workgroup) and an add over split rows
     make = _k_quantized(O.Q4_K, 71)
     gate, up = make(1100, 5120), make(1100, 5120)
-    x = O.Rng(72).floats(6 * 5120)
-    want = O.silu_mul(O.matmul(gate, x), O.matmul(up, x))
-    out, scratch = gpu.alloc(6 * 1100), gpu.alloc(6 * 1100)
-    gpu.swiglu(out, gpu.upload(to_tensor(gate)), gpu.upload(to_tensor(up)), gpu.buffer(x), scratch)
-    close(gpu.read(out), want, 1e-4)
+    gg, gu = gpu.upload(to_tensor(gate)), gpu.upload(to_tensor(up))
+    for n in (2, 3, 4, 6):
+        x = O.Rng(72).floats(n * 5120)
+        want = O.silu_mul(O.matmul(gate, x), O.matmul(up, x))
+        out, scratch = gpu.alloc(n * 1100), gpu.alloc(n * 1100)
+        gpu.swiglu(out, gg, gu, gpu.buffer(x), scratch)
+        close(gpu.read(out), want, 1e-4)
     w = make(300, 17408)
     inp, res = O.Rng(73).floats(4 * 17408), O.Rng(74).floats(4 * 300)
     out = gpu.buffer(res)
@@ -662,6 +664,28 @@ def test_delta_net_chunks_agree_with_the_token_loop_at_full_size(gpu):
         parts.append(gpu.read(o))
     close(gpu.read(out), np.concatenate(parts), 1e-4)
     close(gpu.read(st), gpu.read(want_state), 1e-4)
+
+
+def test_delta_net_past_a_run_of_chunks(gpu):
+    """4096 tokens a pair of launches: one call of 4096 + 70 is, bit for bit,
+    a call of 4096 and one of 70 that goes on from its state."""
+    nk, nv, n, first = 1, 2, 4096 + 70, 4096
+    q, k, v, gates, decay, state = _delta_inputs(O.Rng(15), n, nk, nv)
+    for a in (q, k):
+        r = a.reshape(n * nk, 128)
+        r /= np.sqrt((r.astype(np.float64) ** 2).sum(1, keepdims=True)).astype(np.float32)
+
+    def run(lo, hi, st):
+        out = gpu.alloc((hi - lo) * nv * 128)
+        cut = [a.reshape(n, -1)[lo:hi].ravel() for a in (q, k, v, gates)]
+        gpu.delta_net_unit_keys(out, *(gpu.buffer(a) for a in cut), gpu.buffer(decay), st, nk, nv, 128)
+        return gpu.read(out)
+
+    one, two = gpu.buffer(state), gpu.buffer(state)
+    got = run(0, n, one)
+    want = np.concatenate([run(0, first, two), run(first, n, two)])
+    assert got.tobytes() == want.tobytes()
+    assert gpu.read(one).tobytes() == gpu.read(two).tobytes()
 
 
 def test_argmax_takes_the_first_maximum(gpu):
