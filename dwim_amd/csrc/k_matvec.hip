@@ -173,6 +173,102 @@ static hipError_t launch_vec_bf16(hipStream_t s, const dwim_weight *w, const dwi
     }
 }
 
+// Up to four tokens through a small Q4_0 or Q8_0 matrix: a workgroup takes a tile of 16
+// rows (layout.h), its waves every KW-th unit of 128 columns, lane (kq, c)
+// row c's 16-byte chunks kq, kq + 4: the sums meet by lane swaps and once in LDS.
+// Without the conversion of the activations into LDS that k_rows_few starts
+// with, which is most of its time here.
+template <int FMT, int T>
+__global__ void __launch_bounds__(1024) k_vec_tiles(const uint4 *__restrict__ q, const uint16_t *__restrict__ s,
+                                                    const float *__restrict__ x, float *out, unsigned rows, unsigned cols,
+                                                    int add) {
+    constexpr int L = FMT == DWIM_Q4_0 ? 1 : 2;  // chunks a lane and unit
+    __shared__ float red[16][T][16];
+    const unsigned lane = threadIdx.x & 63, kq = lane >> 4, c = lane & 15, wave = threadIdx.x >> 6, KW = blockDim.x >> 6;
+    const unsigned units = (cols + 127) / 128;
+    const size_t tile = blockIdx.x;
+    float acc[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) acc[t] = 0.0f;
+    for (unsigned u = wave; u < units; u += KW) {
+        const size_t at = tile * units + u;
+        uint4 w[L];
+        uint16_t d[L];
+#pragma unroll
+        for (int i = 0; i < L; i++) {
+            w[i] = q[(at * L + i) * 64 + lane];
+            d[i] = s[(at * 16 + c) * 4 + (L == 1 ? kq : 2 * i + (kq >> 1))];
+        }
+#pragma unroll
+        for (int i = 0; i < L; i++) {
+            const unsigned col = 128 * u + (L == 1 ? 32 * kq : 64 * i + 16 * kq);
+            if (col >= cols) continue;  // (padding)
+            const uint32_t v[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+            const float scale = dq::from_f16(d[i]);
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                const float4 *xt = (const float4 *)(x + (size_t)t * cols + col);
+                float sum = 0.0f;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float4 a = xt[k];
+                    if constexpr (FMT == DWIM_Q4_0) {
+                        const float4 b = xt[4 + k];
+                        auto lo = [&](int e) { return (float)((int)(v[k] >> (8 * e) & 15u) - 8); };
+                        auto hi = [&](int e) { return (float)((int)(v[k] >> (8 * e + 4) & 15u) - 8); };
+                        sum = fmaf(lo(3), a.w, fmaf(lo(2), a.z, fmaf(lo(1), a.y, fmaf(lo(0), a.x, sum))));
+                        sum = fmaf(hi(3), b.w, fmaf(hi(2), b.z, fmaf(hi(1), b.y, fmaf(hi(0), b.x, sum))));
+                    } else {
+                        auto b = [&](int e) { return (float)(int8_t)(v[k] >> (8 * e)); };
+                        sum = fmaf(b(3), a.w, fmaf(b(2), a.z, fmaf(b(1), a.y, fmaf(b(0), a.x, sum))));
+                    }
+                }
+                acc[t] = fmaf(scale, sum, acc[t]);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+        float a, b;
+        xlane::swap16(acc[t], a, b);
+        xlane::swap32(a + b, a, b);
+        if (kq == 0) red[wave][t][c] = a + b;
+    }
+    __syncthreads();
+    const unsigned t = threadIdx.x >> 4, row = (unsigned)tile * 16 + c;
+    if (t >= T || row >= rows) return;
+    float v = 0.0f;
+    for (unsigned k = 0; k < KW; k++) v += red[k][t][c];
+    float *o = out + (size_t)t * rows + row;
+    *o = add ? *o + v : v;
+}
+
+// What goes there: two to four tokens over rows of few units.  Measured on MI355X, us, k_rows_few |
+// here, Q8_0: 1024×1024 2 tokens 4.8 | 3.5, 4 5.0 | 3.9; 4096×1024 4 5.5 | 4.0; 8192×1024
+// 2 5.6 | 4.4, 4 5.5 | 6.1; 100000×1024 2 (from HBM) 40.3 | 39.3, Q4_0 41.5 | 35.0;
+// 2048×2048 2 5.3 | 4.3, 4 5.5 | 6.1; 8192×2048 2 (from HBM) 8.0 | 8.7; 1000×4096
+// 2 6.3 | 6.5.  One token takes no longer there (1024×1024 3.0 | 3.4).
+static bool vec_tiles(const dwim_weight *w, size_t n) {
+    if ((w->fmt != DWIM_Q4_0 && w->fmt != DWIM_Q8_0) || n < 2 || n > 4 || w->rows >= (1u << 31)) return false;
+    return w->cols <= 1024 ? n == 2 || w->rows * n <= 16384 : w->cols <= 2048 && n == 2 && w->rows <= 2048;
+}
+
+template <int FMT>
+static hipError_t launch_vec_tiles(hipStream_t s, const dwim_weight *w, float *out, const float *x, size_t n, int add) {
+    // (the waves' units as even as may be, at most 16 waves)
+    const unsigned units = (unsigned)((w->cols + 127) / 128), each = (units + 15) / 16, kw = (units + each - 1) / each;
+    const unsigned blocks = (unsigned)((w->rows + 15) / 16), threads = 64 * kw;
+    const unsigned rows = (unsigned)w->rows, cols = (unsigned)w->cols;
+    const uint4 *q = (const uint4 *)w->q;
+    const uint16_t *sc = (const uint16_t *)w->s;
+    switch (n) {
+    case 2: k_vec_tiles<FMT, 2><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
+    case 3: k_vec_tiles<FMT, 3><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
+    default: k_vec_tiles<FMT, 4><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
+    }
+    return hipGetLastError();
+}
+
 // The most tokens that go through the kernel that converts the activations
 // itself (k_rows_few.hip); more go through the GEMM (k_gemm_rows.hip), whose
 // split of the activations and sum of the parts are launches of their own.
@@ -202,6 +298,12 @@ hipError_t launch_rows(dwim_dev *dev, const dwim_weight *w, const dwim_weight *u
         const size_t m = std::min(most, n - t);
         float *const o = out + t * w->rows;
         const float *const xt = x + t * w->cols;
+        if (!up && vec_tiles(w, m)) {
+            const hipError_t e = w->fmt == DWIM_Q4_0 ? launch_vec_tiles<DWIM_Q4_0>(dev->stream, w, o, xt, m, add)
+                                                     : launch_vec_tiles<DWIM_Q8_0>(dev->stream, w, o, xt, m, add);
+            if (e != hipSuccess) return e;
+            continue;
+        }
         const hipError_t e = w->fmt == DWIM_BF16 && m <= kVecTokens ? launch_vec_bf16(dev->stream, w, up, o, xt, m, add)
                                                                      : launch_rows_few(dev, w, up, o, xt, m, add);
         if (e != hipSuccess) return e;

@@ -93,6 +93,21 @@ def test_swiglu_pair(gpu, name, rows, cols, n):
     assert (np.abs(gpu.read(out).reshape(n, rows) - want) <= bound).all()
 
 
+@pytest.mark.parametrize("name", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("rows,cols,n", [(5461, 1024, 3), (5462, 1024, 3), (4096, 1024, 4), (4097, 992, 4), (16, 32, 2), (9000, 160, 2),
+                                         (2048, 2048, 2), (2049, 2048, 2), (37, 1056, 2), (50, 2080, 2), (17, 1056, 3)])
+def test_few_tokens_of_few_units(gpu, name, rows, cols, n):
+    """Both sides of the rule that takes two to four tokens over short rows to
+    the vector ALUs; whole and part units, one wave to 16."""
+    t, w = weight(name, rows, cols, 9)
+    x, base = O.Rng(n).floats(n * cols).reshape(n, cols), O.Rng(n + 1).floats(n * rows)
+    gw, gx, out, acc = gpu.upload(t), gpu.buffer(x), gpu.alloc(n * rows), gpu.buffer(base)
+    gpu.matmul(out, gw, gx)
+    check(gpu.read(out), w, x)
+    gpu.matmul_add(acc, gw, gx, gpu.alloc(n * rows))
+    check(gpu.read(acc), w, x, base.reshape(n, rows).astype(np.float64))
+
+
 @pytest.mark.parametrize("rows,cols", [(16383, 24), (16384, 520), (16387, 40)])
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5])
 def test_bf16_of_many_rows(gpu, rows, cols, n):
