@@ -284,7 +284,10 @@ __global__ void __launch_bounds__(kPThreads) k_attn_partial(float *__restrict__ 
 //     hi and lo parts, as A against the values as B (transposed into LDS,
 //     8 positions of one dimension a lane).
 // Every product is exact up to the hi/lo split (2^-22 relative) and summed
-// in f32.
+// in f32.  WIDE (batches, over Q8 caches): the values' scales of a step and Q8 block are
+// taken times a power of two that brings the largest to [2^14, 2^15), so that
+// no probability times a scale is small in f16 (small ones cost 6e-6 of the
+// result; k_attn_flash 4e-7), and a step's products are summed by themselves.
 constexpr int kMStep = 64;       // positions a step
 constexpr int kMThreads = 256;
 constexpr int kQStride = 256 + 8;  // halfs a staged query row (bank spread)
@@ -313,7 +316,7 @@ constexpr size_t mfma_lds(int rt, bool f16) {
            (size_t)16 * rt * 3 * 4 + (size_t)kMStep * (f16 ? kVRow16 : kVRow);
 }
 
-template <int RT, bool F16>
+template <int RT, bool F16, bool WIDE>
 __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ partials, const float *__restrict__ q,
                                                          const int8_t *__restrict__ kq,
                                                          const uint16_t *__restrict__ ks,
@@ -323,6 +326,7 @@ __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ 
     constexpr int NR = 16 * RT;  // rows, padded
     constexpr int D = kFD;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
+    __shared__ float unscale[WIDE ? 8 : 1];  // of a step's scales, by Q8 block
     _Float16 *q_hi = (_Float16 *)lds_raw, *q_lo = q_hi + NR * kQStride;
     float *p_s = (float *)(q_lo + NR * kQStride);
     float(*vsc_s)[kMStep] = (float(*)[kMStep])(p_s + NR * kPStride);
@@ -431,7 +435,17 @@ __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ 
             if (threadIdx.x < kMStep) {
                 const uint32_t w4[4] = {vscale.x, vscale.y, vscale.z, vscale.w};
 #pragma unroll
-                for (int b = 0; b < 8; b++) vsc_s[b][threadIdx.x] = dq::from_f16((uint16_t)(w4[b / 2] >> (16 * (b % 2))));
+                for (int b = 0; b < 8; b++) {
+                    const float d = dq::from_f16((uint16_t)(w4[b / 2] >> (16 * (b % 2))));
+                    float up = 1.0f;
+                    if constexpr (WIDE) {  // (wave 0)
+                        const float top = group_max<64>(fabsf(d));
+                        const int sh2 = top > 0.0f ? 141 - (int)(__float_as_uint(top) >> 23) : 0;
+                        up = __uint_as_float((unsigned)(sh2 + 127) << 23);
+                        if (lane == 0) unscale[b] = __uint_as_float((unsigned)(127 - sh2) << 23);
+                    }
+                    vsc_s[b][threadIdx.x] = d * up;
+                }
             }
         }
         if (next) load_values(pn, count(pn));
@@ -506,6 +520,12 @@ __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ 
 #pragma unroll
                 for (int e = 0; e < 4; e++) o[rt][j][e] *= a[e];
         }
+        afloat4 part[WIDE ? RT : 1][WIDE ? 4 : 1];  // this step's
+        if constexpr (WIDE)
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) part[rt][j] = afloat4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int k2 = 0; k2 < 2; k2++) {
             const int pp = 32 * k2 + 8 * kq4;  // this lane's 8 positions
@@ -553,7 +573,12 @@ __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ 
                     ahalf8 ph, pl;
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
-                        const float x = F16 ? pr[i] : pr[i] * vsc_s[2 * wave + h][pp + i];
+                        float x = F16 ? pr[i] : pr[i] * vsc_s[2 * wave + h][pp + i];
+                        // (one product: left to itself the compiler rounds hi from
+                        // it, and lo from the exact product less another hi, which
+                        // differ now and then: 5e-6 of the results, and 1% of the
+                        // time of a token at 32k positions)
+                        if (WIDE) asm volatile("" : "+v"(x));
                         const _Float16 hh = (_Float16)x;
                         ph[i] = hh;
                         pl[i] = (_Float16)(x - (float)hh);
@@ -561,12 +586,22 @@ __global__ void __launch_bounds__(kMThreads, 2) k_attn_mfma(float *__restrict__ 
 #pragma unroll
                     for (int jj = 0; jj < 2; jj++) {
                         const int j = 2 * h + jj;
-                        o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb[j], o[rt][j], 0, 0, 0);
-                        o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb[j], o[rt][j], 0, 0, 0);
+                        afloat4 &to = WIDE ? part[WIDE ? rt : 0][WIDE ? j : 0] : o[rt][j];
+                        to = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb[j], to, 0, 0, 0);
+                        to = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb[j], to, 0, 0, 0);
                     }
                 }
             }
         }
+        if constexpr (WIDE)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float down = unscale[2 * wave + j / 2];
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[rt][j][e] = fmaf(part[rt][j][e], down, o[rt][j][e]);
+            }
     }
     // ---- the partial rows: row 4·kq4 + e of tile rt, dimension 64w + 16j + r16
 #pragma unroll
@@ -1075,10 +1110,9 @@ unsigned flash_parts(const dwim_dev *dev, size_t n, size_t pos, size_t n_heads, 
 // once.  There is no cache to expand then, and none of what a block of
 // k_attn_flash does once (its queries, a prologue of two steps, the scores of
 // the step past the last), most of its time when the steps are few.  Measured on
-// MI355X (us, flash | so), 24 / 4 heads, q8: 16 tokens at position 0 16.4 | 12, at
-// 100 23 | 13, at 1000 35 | 22, at 4000 (past the blocks' limit) 40 | 36; 32 at 0 17.6 | 16, at
-// 200 32 | 18.  The pass takes 0.2 us more a token (its merge): 64 at 0 20 | 24,
-// hence the limit of rows.
+// MI355X (us, flash | so), 24 / 4 heads, q8: 16 tokens at position 0 16.4 | 13.6, at
+// 100 23 | 14, at 1000 35 | 22.5; 32 at 0 17.6 | 16.7, at 200 32 | 19.  The pass takes
+// 0.2 us more a token (its merge): 64 at 0 20 | 24, hence the limit of rows.
 constexpr size_t kShortRows = 768;
 size_t short_batch_tokens(const dwim_dev *dev, size_t n, size_t pos, size_t n_heads, size_t n_kv_heads) {
     const size_t G = n_heads / n_kv_heads, slots = kMPerCU * (size_t)dev->cus;
@@ -1116,15 +1150,15 @@ namespace {
 // 32k: 47.8 against 31.2)
 constexpr size_t kValuLen = 6144;
 
-template <int RT, bool F16>
+template <int RT, bool F16, bool WIDE>
 hipError_t mfma_pass(dwim_dev *dev, dim3 grid, float *partials, const float *q, const dwim_cache *k,
                      const dwim_cache *v, const Shape &sh, int G, int T, float qscale) {
     constexpr size_t lds = mfma_lds(RT, F16);
     // once a process (thread-safe: a function-local static)
     static const hipError_t raised =
-        hipFuncSetAttribute((const void *)k_attn_mfma<RT, F16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipFuncSetAttribute((const void *)k_attn_mfma<RT, F16, WIDE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (raised != hipSuccess) return raised;
-    k_attn_mfma<RT, F16><<<grid, kMThreads, lds, dev->stream>>>(partials, q, k->q, k->s, v->q, v->s, sh, G, T, qscale);
+    k_attn_mfma<RT, F16, WIDE><<<grid, kMThreads, lds, dev->stream>>>(partials, q, k->q, k->s, v->q, v->s, sh, G, T, qscale);
     return hipGetLastError();
 }
 
@@ -1185,10 +1219,9 @@ hipError_t attention_run(dwim_dev *dev, float *partials, float *out, const float
         const size_t ch = kMStep * std::max<size_t>(1, (base + slots - 1) / slots), chunks = (len + ch - 1) / ch;
         Shape sh{n, pos, n_heads, head_dim, n_kv_heads, ch, chunks};
         dim3 g1((unsigned)chunks, (unsigned)n_kv_heads, (unsigned)groups);
-        hipError_t e = T * G <= 16 ? (k->f16 ? mfma_pass<1, true>(dev, g1, partials, q, k, v, sh, G, T, qscale)
-                                             : mfma_pass<1, false>(dev, g1, partials, q, k, v, sh, G, T, qscale))
-                                   : (k->f16 ? mfma_pass<2, true>(dev, g1, partials, q, k, v, sh, G, T, qscale)
-                                             : mfma_pass<2, false>(dev, g1, partials, q, k, v, sh, G, T, qscale));
+        auto pass = T * G <= 16 ? (k->f16 ? mfma_pass<1, true, false> : few ? mfma_pass<1, false, true> : mfma_pass<1, false, false>)
+                                : (k->f16 ? mfma_pass<2, true, false> : few ? mfma_pass<2, false, true> : mfma_pass<2, false, false>);
+        hipError_t e = pass(dev, g1, partials, q, k, v, sh, G, T, qscale);
         if (e != hipSuccess) return e;
         dim3 g2((unsigned)n_heads * (unsigned)(head_dim / 64), (unsigned)n);
         k_attn_combine<<<g2, kCThreads, 0, dev->stream>>>(out, partials, sh, gate, pv);

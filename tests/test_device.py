@@ -748,3 +748,34 @@ def test_attention_batch_edges_against_float64(gpu, heads, kv, n, pos, f16):
         ds = (256 * 2.0**-24 + 2.0**-20) * size.max(1, keepdims=True)
         bound = (2 * ds + 2.0**-20 + (64 + length) * 2.0**-24) * (p @ np.abs(vh))
         assert (np.abs(got[:, h] - p @ vh) <= bound).all(), h
+
+
+@pytest.mark.parametrize("heads,kv,n,pos", [(16, 8, 16, 100), (24, 4, 16, 1000), (24, 4, 24, 20), (8, 1, 40, 300), (32, 32, 17, 0),
+                                            (24, 4, 48, 100)])
+def test_attention_batches_over_a_q8_cache_keep_their_bits(gpu, heads, kv, n, pos):
+    """A probability times a value's scale (here 1/64 and below) is small in f16,
+    and its two parts must come of one rounding: short batches had 5e-6 of error
+    without either, with both 4e-7, as the batch kernel.  The parts keep 2^-22 of a
+    probability, a score 2^-22 of itself and of up to 40: 40 · 2^-22 / sqrt(256) and
+    the sums' roundings stay under 1e-6."""
+    rng = np.random.default_rng(heads + n + pos)
+    length, d = pos + n, 256
+    k, v = (rng.integers(-127, 128, (length, kv, d)).astype(np.float32) / s for s in (64, 8192))
+    for a, s in ((k, 64), (v, 8192)):
+        a[..., ::32] = np.float32(127 / s)
+    q = rng.standard_normal((n, heads, d), dtype=np.float32)
+    caches = []
+    for a in (k, v):
+        c = gpu.alloc_cache(a.size)
+        gpu.store(c, 0, gpu.buffer(a.ravel()))
+        caches.append(c)
+    out = gpu.alloc(q.size)
+    gpu.attention(out, gpu.buffer(q.ravel()), *caches, pos, heads, d, kv)
+    got = gpu.read(out).reshape(n, heads, d)
+    want = np.empty((n, heads, d))
+    for h in range(heads):
+        s = q[:, h].astype(np.float64) @ k[:, h // (heads // kv)].astype(np.float64).T / 16
+        s = np.where(np.arange(length)[None] <= pos + np.arange(n)[:, None], s, -np.inf)
+        p = np.exp(s - s.max(1, keepdims=True))
+        want[:, h] = p / p.sum(1, keepdims=True) @ v[:, h // (heads // kv)].astype(np.float64)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
