@@ -18,7 +18,8 @@
 //
 // A batch of 16 tokens or more (head_dim 256) runs flash attention on the
 // f16 matrix cores over a copy of the cache expanded to f16 hi + lo parts in
-// the layout the kernel holds in LDS (k_kv_expand, k_attn_flash below).
+// the layout the kernel holds in LDS (k_kv_expand, k_attn_flash below), but for
+// short ones (short_batch_tokens), which take the decode pass of k_attn_mfma.
 #include "device_util.h"
 #include "planes.h"
 #include "quant_math.h"
