@@ -173,53 +173,57 @@ static hipError_t launch_vec_bf16(hipStream_t s, const dwim_weight *w, const dwi
     }
 }
 
-// Up to four tokens through a small Q4_0 or Q8_0 matrix: a workgroup takes a tile of 16
-// rows (layout.h), its waves every KW-th unit of 128 columns, lane (kq, c)
-// row c's 16-byte chunks kq, kq + 4: the sums meet by lane swaps and once in LDS.
-// Without the conversion of the activations into LDS that k_rows_few starts
-// with, which is most of its time here.
-template <int FMT, int T>
+// Up to four tokens through a small Q4_0 or Q8_0 matrix: a workgroup takes RR rows
+// of a tile of 16 (layout.h: chunk m of a row lies 256 bytes after chunk m - 1), a wave
+// U × 64 / RR chunks of each at a time, lane (g, c) row c's chunks g, g + 64 / RR, ..;
+// the sums meet by lane swaps and once in LDS.  Without the conversion of the activations
+// into LDS that k_rows_few starts with, which is most of its time here, and with
+// RR = 4 four times its workgroups.
+constexpr unsigned vec_loads(int fmt, int rr) { return rr == 16 && fmt == DWIM_Q4_0 ? 1 : 2; }  // U: 8 waves at 1024 columns
+
+template <int FMT, int T, int RR>
 __global__ void __launch_bounds__(1024) k_vec_tiles(const uint4 *__restrict__ q, const uint16_t *__restrict__ s,
                                                     const float *__restrict__ x, float *out, unsigned rows, unsigned cols,
                                                     int add) {
-    constexpr int L = FMT == DWIM_Q4_0 ? 1 : 2;  // chunks a lane and unit
-    __shared__ float red[16][T][16];
-    const unsigned lane = threadIdx.x & 63, kq = lane >> 4, c = lane & 15, wave = threadIdx.x >> 6, KW = blockDim.x >> 6;
-    const unsigned units = (cols + 127) / 128;
-    const size_t tile = blockIdx.x;
+    constexpr unsigned G = 64 / RR, U = vec_loads(FMT, RR), kWeights = FMT == DWIM_Q4_0 ? 32 : 16, kPer = 128 / kWeights;
+    __shared__ float red[16][T][RR];
+    const unsigned lane = threadIdx.x & 63, g = lane / RR, c = lane % RR, wave = threadIdx.x >> 6, KW = blockDim.x >> 6;
+    const unsigned units = (cols + 127) / 128, chunks = cols / kWeights;
+    const unsigned row0 = blockIdx.x * RR, in_tile = row0 % 16 + c;
+    const size_t base = (size_t)(row0 / 16) * units;
     float acc[T];
 #pragma unroll
     for (int t = 0; t < T; t++) acc[t] = 0.0f;
-    for (unsigned u = wave; u < units; u += KW) {
-        const size_t at = tile * units + u;
-        uint4 w[L];
-        uint16_t d[L];
+    for (unsigned m0 = wave * U * G; m0 < chunks; m0 += KW * U * G) {
+        uint4 w[U];
+        uint16_t d[U];
 #pragma unroll
-        for (int i = 0; i < L; i++) {
-            w[i] = q[(at * L + i) * 64 + lane];
-            d[i] = s[(at * 16 + c) * 4 + (L == 1 ? kq : 2 * i + (kq >> 1))];
+        for (unsigned i = 0; i < U; i++) {  // (past the row's chunks the last one's, unused)
+            const unsigned m = min(m0 + i * G + g, chunks - 1), b = m * kWeights / 32;
+            w[i] = q[(base * kPer + m) * 16 + in_tile];
+            d[i] = s[((base + b / 4) * 16 + in_tile) * 4 + b % 4];
         }
 #pragma unroll
-        for (int i = 0; i < L; i++) {
-            const unsigned col = 128 * u + (L == 1 ? 32 * kq : 64 * i + 16 * kq);
-            if (col >= cols) continue;  // (padding)
+        for (unsigned i = 0; i < U; i++) {
+            const unsigned m = m0 + i * G + g;
+            if (m >= chunks) continue;
             const uint32_t v[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
             const float scale = dq::from_f16(d[i]);
 #pragma unroll
             for (int t = 0; t < T; t++) {
-                const float4 *xt = (const float4 *)(x + (size_t)t * cols + col);
+                const float4 *xt = (const float4 *)(x + (size_t)t * cols + m * kWeights);
                 float sum = 0.0f;
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const float4 a = xt[k];
                     if constexpr (FMT == DWIM_Q4_0) {
-                        const float4 b = xt[4 + k];
-                        auto lo = [&](int e) { return (float)((int)(v[k] >> (8 * e) & 15u) - 8); };
-                        auto hi = [&](int e) { return (float)((int)(v[k] >> (8 * e + 4) & 15u) - 8); };
+                        const float4 e = xt[4 + k];
+                        auto lo = [&](int j) { return (float)((int)(v[k] >> (8 * j) & 15u) - 8); };
+                        auto hi = [&](int j) { return (float)((int)(v[k] >> (8 * j + 4) & 15u) - 8); };
                         sum = fmaf(lo(3), a.w, fmaf(lo(2), a.z, fmaf(lo(1), a.y, fmaf(lo(0), a.x, sum))));
-                        sum = fmaf(hi(3), b.w, fmaf(hi(2), b.z, fmaf(hi(1), b.y, fmaf(hi(0), b.x, sum))));
+                        sum = fmaf(hi(3), e.w, fmaf(hi(2), e.z, fmaf(hi(1), e.y, fmaf(hi(0), e.x, sum))));
                     } else {
-                        auto b = [&](int e) { return (float)(int8_t)(v[k] >> (8 * e)); };
+                        auto b = [&](int j) { return (float)(int8_t)(v[k] >> (8 * j)); };
                         sum = fmaf(b(3), a.w, fmaf(b(2), a.z, fmaf(b(1), a.y, fmaf(b(0), a.x, sum))));
                     }
                 }
@@ -229,42 +233,52 @@ __global__ void __launch_bounds__(1024) k_vec_tiles(const uint4 *__restrict__ q,
     }
 #pragma unroll
     for (int t = 0; t < T; t++) {
-        float a, b;
-        xlane::swap16(acc[t], a, b);
+        float v = acc[t], a, b;
+        if (RR == 4) {  // (rotations of 16 lanes by 4 and 8)
+            v += xlane::mov<0x124>(v);
+            v += xlane::mov<0x128>(v);
+        }
+        xlane::swap16(v, a, b);
         xlane::swap32(a + b, a, b);
-        if (kq == 0) red[wave][t][c] = a + b;
+        if (g == 0) red[wave][t][c] = a + b;
     }
     __syncthreads();
-    const unsigned t = threadIdx.x >> 4, row = (unsigned)tile * 16 + c;
+    const unsigned t = threadIdx.x / RR, row = row0 + threadIdx.x % RR;
     if (t >= T || row >= rows) return;
     float v = 0.0f;
-    for (unsigned k = 0; k < KW; k++) v += red[k][t][c];
+    for (unsigned k = 0; k < KW; k++) v += red[k][t][threadIdx.x % RR];
     float *o = out + (size_t)t * rows + row;
     *o = add ? *o + v : v;
 }
 
-// What goes there: two to four tokens over rows of few units.  Measured on MI355X, us, k_rows_few |
-// here, Q8_0: 1024×1024 2 tokens 4.8 | 3.5, 4 5.0 | 3.9; 4096×1024 4 5.5 | 4.0; 8192×1024
-// 2 5.6 | 4.4, 4 5.5 | 6.1; 100000×1024 2 (from HBM) 40.3 | 39.3, Q4_0 41.5 | 35.0;
-// 2048×2048 2 5.3 | 4.3, 4 5.5 | 6.1; 8192×2048 2 (from HBM) 8.0 | 8.7; 1000×4096
-// 2 6.3 | 6.5.  One token takes no longer there (1024×1024 3.0 | 3.4).
-static bool vec_tiles(const dwim_weight *w, size_t n) {
-    if ((w->fmt != DWIM_Q4_0 && w->fmt != DWIM_Q8_0) || n < 2 || n > 4 || w->rows >= (1u << 31)) return false;
-    return w->cols <= 1024 ? n == 2 || w->rows * n <= 16384 : w->cols <= 2048 && n == 2 && w->rows <= 2048;
+// What goes there: two to four tokens over rows of few units (RR = 16), one over
+// few rows (RR = 4).  Measured on MI355X, us, k_rows_few | here, Q8_0: 1024×1024 2
+// tokens 4.8 | 3.5, 4 5.0 | 3.9; 4096×1024 4 5.5 | 4.0; 8192×1024 2 5.6 | 4.4, 4 5.5 |
+// 6.1; 100000×1024 2 (from HBM) 40.3 | 39.3, Q4_0 41.5 | 35.0; 2048×2048 2 5.3 | 4.3, 4
+// 5.5 | 6.1; 8192×2048 2 (from HBM) 8.0 | 8.7; 1000×4096 2 6.3 | 6.5; one token 96×5120 5.2 |
+// 3.4, 1024×5120 5.3 | 3.0 (from HBM 5.6 | 4.7), 1024×17408 12.7 | 8.4, 1024×2048 3.4 |
+// 3.2, 2048×5120 from HBM 5.9 | 6.4 (a line is read by two workgroups).
+static int vec_tiles(const dwim_weight *w, size_t n) {
+    if ((w->fmt != DWIM_Q4_0 && w->fmt != DWIM_Q8_0) || n > 4 || w->rows >= (1u << 31) || w->cols >= (1u << 31)) return 0;
+    if (n == 1) return w->rows <= 1024 && w->cols > 2048 ? 4 : 0;
+    return (w->cols <= 1024 ? n == 2 || w->rows * n <= 16384 : w->cols <= 2048 && n == 2 && w->rows <= 2048) ? 16 : 0;
 }
 
 template <int FMT>
-static hipError_t launch_vec_tiles(hipStream_t s, const dwim_weight *w, float *out, const float *x, size_t n, int add) {
-    // (the waves' units as even as may be, at most 16 waves)
-    const unsigned units = (unsigned)((w->cols + 127) / 128), each = (units + 15) / 16, kw = (units + each - 1) / each;
-    const unsigned blocks = (unsigned)((w->rows + 15) / 16), threads = 64 * kw;
+static hipError_t launch_vec_tiles(hipStream_t s, const dwim_weight *w, float *out, const float *x, size_t n, int add,
+                                   int rr) {
+    // (the waves' steps as even as may be, at most 16 waves)
+    const size_t step = (size_t)64 / rr * vec_loads(FMT, rr) * (FMT == DWIM_Q4_0 ? 32 : 16);
+    const unsigned steps = (unsigned)((w->cols + step - 1) / step), each = (steps + 15) / 16, kw = (steps + each - 1) / each;
+    const unsigned blocks = (unsigned)((w->rows + rr - 1) / rr), threads = 64 * kw;
     const unsigned rows = (unsigned)w->rows, cols = (unsigned)w->cols;
     const uint4 *q = (const uint4 *)w->q;
     const uint16_t *sc = (const uint16_t *)w->s;
     switch (n) {
-    case 2: k_vec_tiles<FMT, 2><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
-    case 3: k_vec_tiles<FMT, 3><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
-    default: k_vec_tiles<FMT, 4><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
+    case 1: k_vec_tiles<FMT, 1, 4><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
+    case 2: k_vec_tiles<FMT, 2, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
+    case 3: k_vec_tiles<FMT, 3, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
+    default: k_vec_tiles<FMT, 4, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
     }
     return hipGetLastError();
 }
@@ -298,9 +312,9 @@ hipError_t launch_rows(dwim_dev *dev, const dwim_weight *w, const dwim_weight *u
         const size_t m = std::min(most, n - t);
         float *const o = out + t * w->rows;
         const float *const xt = x + t * w->cols;
-        if (!up && vec_tiles(w, m)) {
-            const hipError_t e = w->fmt == DWIM_Q4_0 ? launch_vec_tiles<DWIM_Q4_0>(dev->stream, w, o, xt, m, add)
-                                                     : launch_vec_tiles<DWIM_Q8_0>(dev->stream, w, o, xt, m, add);
+        if (const int rr = up ? 0 : vec_tiles(w, m)) {
+            const hipError_t e = w->fmt == DWIM_Q4_0 ? launch_vec_tiles<DWIM_Q4_0>(dev->stream, w, o, xt, m, add, rr)
+                                                     : launch_vec_tiles<DWIM_Q8_0>(dev->stream, w, o, xt, m, add, rr);
             if (e != hipSuccess) return e;
             continue;
         }
