@@ -251,16 +251,17 @@ __global__ void __launch_bounds__(1024) k_vec_tiles(const uint4 *__restrict__ q,
     *o = add ? *o + v : v;
 }
 
-// What goes there: two to four tokens over rows of few units (RR = 16), one over
-// few rows (RR = 4).  Measured on MI355X, us, k_rows_few | here, Q8_0: 1024×1024 2
+// What goes there: two to four tokens over rows of few units (RR = 16), one to four
+// over few long rows (RR = 4), whose tiles are too few for k_rows_few.  Measured on MI355X, us, k_rows_few | here, Q8_0: 1024×1024 2
 // tokens 4.8 | 3.5, 4 5.0 | 3.9; 4096×1024 4 5.5 | 4.0; 8192×1024 2 5.6 | 4.4, 4 5.5 |
 // 6.1; 100000×1024 2 (from HBM) 40.3 | 39.3, Q4_0 41.5 | 35.0; 2048×2048 2 5.3 | 4.3, 4
 // 5.5 | 6.1; 8192×2048 2 (from HBM) 8.0 | 8.7; 1000×4096 2 6.3 | 6.5; one token 96×5120 5.2 |
-// 3.4, 1024×5120 5.3 | 3.0 (from HBM 5.6 | 4.7), 1024×17408 12.7 | 8.4, 1024×2048 3.4 |
-// 3.2, 2048×5120 from HBM 5.9 | 6.4 (a line is read by two workgroups).
+// 3.3, 1024×5120 5.3 | 3.0 (from HBM 5.5 | 4.8; 4 tokens 10.2 | 6.4), 1024×17408 12.7 | 8.6,
+// 1024×2048 3.4 | 3.2, 2048×5120 from HBM 5.9 | 6.4 (a line is read by two workgroups).
 static int vec_tiles(const dwim_weight *w, size_t n) {
     if ((w->fmt != DWIM_Q4_0 && w->fmt != DWIM_Q8_0) || n > 4 || w->rows >= (1u << 31) || w->cols >= (1u << 31)) return 0;
-    if (n == 1) return w->rows <= 1024 && w->cols > 2048 ? 4 : 0;
+    if (w->rows <= 1024 && w->cols > 2048) return 4;
+    if (n == 1) return 0;
     return (w->cols <= 1024 ? n == 2 || w->rows * n <= 16384 : w->cols <= 2048 && n == 2 && w->rows <= 2048) ? 16 : 0;
 }
 
@@ -276,9 +277,18 @@ static hipError_t launch_vec_tiles(hipStream_t s, const dwim_weight *w, float *o
     const uint16_t *sc = (const uint16_t *)w->s;
     switch (n) {
     case 1: k_vec_tiles<FMT, 1, 4><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
-    case 2: k_vec_tiles<FMT, 2, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
-    case 3: k_vec_tiles<FMT, 3, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
-    default: k_vec_tiles<FMT, 4, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add); break;
+    case 2:
+        if (rr == 4) k_vec_tiles<FMT, 2, 4><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add);
+        else k_vec_tiles<FMT, 2, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add);
+        break;
+    case 3:
+        if (rr == 4) k_vec_tiles<FMT, 3, 4><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add);
+        else k_vec_tiles<FMT, 3, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add);
+        break;
+    default:
+        if (rr == 4) k_vec_tiles<FMT, 4, 4><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add);
+        else k_vec_tiles<FMT, 4, 16><<<blocks, threads, 0, s>>>(q, sc, x, out, rows, cols, add);
+        break;
     }
     return hipGetLastError();
 }

@@ -96,10 +96,11 @@ def test_swiglu_pair(gpu, name, rows, cols, n):
 @pytest.mark.parametrize("name", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("rows,cols,n", [(5461, 1024, 3), (5462, 1024, 3), (4096, 1024, 4), (4097, 992, 4), (16, 32, 2), (9000, 160, 2),
                                          (2048, 2048, 2), (2049, 2048, 2), (37, 1056, 2), (50, 2080, 2), (17, 1056, 3),
-                                         (1, 2080, 1), (18, 4096, 1), (1023, 2176, 1), (1025, 2176, 1), (7, 17408, 1), (30, 16416, 1)])
+                                         (1, 2080, 1), (18, 4096, 1), (1023, 2176, 1), (1025, 2176, 1), (7, 17408, 1), (30, 16416, 1),
+                                         (1024, 2080, 2), (5, 5120, 3), (97, 2336, 4), (1025, 2080, 4)])
 def test_few_tokens_of_few_units(gpu, name, rows, cols, n):
-    """Both sides of the rules that take two to four tokens over short rows, and one
-    over few rows, to the vector ALUs; whole and part units, one wave to 16."""
+    """Both sides of the rules that take two to four tokens over short rows, and up
+    to four over few long ones, to the vector ALUs; whole and part units, one wave to 16."""
     t, w = weight(name, rows, cols, 9)
     x, base = O.Rng(n).floats(n * cols).reshape(n, cols), O.Rng(n + 1).floats(n * rows)
     gw, gx, out, acc = gpu.upload(t), gpu.buffer(x), gpu.alloc(n * rows), gpu.buffer(base)
