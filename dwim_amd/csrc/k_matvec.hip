@@ -300,10 +300,14 @@ static hipError_t launch_vec_tiles(hipStream_t s, const dwim_weight *w, float *o
 // 44, at 32 66 | 48; Q8_0 at 16 53 | 53, at 32 79 | 57; Q6_K at 16 56 | 72, at 32 93
 // | 76; bf16 at 32 113 | 121, at 64 254 | 139; a 2304×3072 Q8_0 pair at 32 17.5 | 17.8,
 // at 64 32 | 24; 5120×17408 Q4_0 at 16 32 | 47, at 32 44 | 48, at 64 75 | 68; Q6_K,
-// whose GEMM scales every 16 columns, at 64 93 | 116; 1024×1024 Q4_0 at 64 12 | 15.
+// whose GEMM scales every 16 columns, at 64 92 | 117, 5120×5120 35 | 45, but with rows
+// for whole rounds of tiles 17408×5120 86 | 59, 20000×2048 44 | 39, 100000×1024 117 | 60;
+// bf16 at 32 5120×5120 31 | 34, 17408×5120 70 | 62; 1024×1024 Q4_0 at 64 12 | 15.
 static size_t few_tokens(const dwim_weight *w, bool pair) {
     const bool small = w->rows * w->cols <= (size_t)8 << 20;
-    if (!pair && (small || w->fmt == DWIM_Q6_K)) return 64;
+    const bool many = w->rows > 8192;
+    if (!pair && (small || w->fmt == DWIM_Q6_K)) return !small && many ? 32 : 64;
+    if (!pair && many && w->fmt == DWIM_BF16) return 16;
     return small || w->fmt == DWIM_BF16 || w->cols >= 2 * w->rows ? 32 : 16;
 }
 

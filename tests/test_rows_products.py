@@ -93,6 +93,18 @@ def test_swiglu_pair(gpu, name, rows, cols, n):
     assert (np.abs(gpu.read(out).reshape(n, rows) - want) <= bound).all()
 
 
+@pytest.mark.parametrize("name,n", [("q6_k", 33), ("q6_k", 64), ("bf16", 17), ("bf16", 32)])
+@pytest.mark.parametrize("rows,cols", [(8192, 1280), (8193, 1280)])
+def test_both_sides_of_many_rows(gpu, name, n, rows, cols):
+    """The few-token kernel and the batch kernel where matrices of many rows change
+    from the one to the other."""
+    t, w = weight(name, rows, cols, 9)
+    x, base = O.Rng(n).floats(n * cols).reshape(n, cols), O.Rng(n + 1).floats(n * rows)
+    acc = gpu.buffer(base)
+    gpu.matmul_add(acc, gpu.upload(t), gpu.buffer(x), gpu.alloc(n * rows))
+    check(gpu.read(acc), w, x, base.reshape(n, rows).astype(np.float64))
+
+
 @pytest.mark.parametrize("name", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("rows,cols,n", [(5461, 1024, 3), (5462, 1024, 3), (4096, 1024, 4), (4097, 992, 4), (16, 32, 2), (9000, 160, 2),
                                          (2048, 2048, 2), (2049, 2048, 2), (37, 1056, 2), (50, 2080, 2), (17, 1056, 3),
